@@ -134,8 +134,10 @@ mk_status mk_stream_create(void** s)
 
 mk_status mk_stream_destroy(void* s)
 {
-    if (s)
+    if (s) {
+        gemm_release_stream(s);
         MK_HIP(hipStreamDestroy(static_cast<hipStream_t>(s)));
+    }
     return MK_OK;
 }
 

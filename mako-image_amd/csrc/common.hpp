@@ -65,6 +65,9 @@ double gemm_cost(const mk_gemm_args* a, uint32_t n, uint32_t cus);
 // MK_ERR_DEVICE when a stream-K launch on `stream` (all: on any stream of any device) gave up waiting for a partial
 // tile since the last check (the check clears it); called after synchronisations of that stream (all: of the device).
 mk_status gemm_take_error(const void* stream, bool all = false);
+// To be called before a stream is destroyed: waits for its last stream-K launch and frees that launch's workspace for
+// other streams (an event must not be asked after the stream it was recorded on is gone).
+void gemm_release_stream(const void* stream);
 
 // ---- ln_modulate over one or two problems in one launch (kernels.hip; the engine groups the two streams) ----
 struct LnArgs {

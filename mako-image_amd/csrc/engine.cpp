@@ -1042,6 +1042,7 @@ mk_status mk_engine_destroy(mk_engine* e)
         (void)hipEventDestroy(e->ord_out);
     if (e->side)
         (void)hipStreamDestroy(e->side);
+    gemm_release_stream(e->stream);
     (void)hipStreamDestroy(e->stream);
     delete e;
     return MK_OK;

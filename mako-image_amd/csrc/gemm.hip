@@ -1484,6 +1484,7 @@ struct SkWork {
     uint32_t nflags = 0, epoch = 0;
     hipStream_t last = nullptr;
     hipEvent_t done = nullptr;
+    bool idle = false; // its last launch's stream is gone, the launch complete: `done` names a dead stream, not asked
     uint64_t used = 0; // launch counter at its last use (least recently used first)
 };
 struct SkDevice {
@@ -1500,6 +1501,19 @@ std::mutex g_sk_mutex;
 SkDevice g_sk[kMaxDevices];
 uint32_t g_sk_polls = kSkPollsDefault;
 
+// Whether a workspace's last launch has completed. The event's state lies with the stream it was recorded on: a
+// stream that a caller destroyed behind the library's back makes the query fail, and that error would otherwise be
+// reported by the next launch (such a workspace counts as busy).
+bool sk_done(const SkWork& w)
+{
+    if (w.idle)
+        return true;
+    const hipError_t e = hipEventQuery(w.done);
+    if (e != hipSuccess && e != hipErrorNotReady)
+        (void)hipGetLastError();
+    return e == hipSuccess;
+}
+
 // A workspace for one stream-K launch of `need` partial bytes on stream s (g_sk_mutex held).
 mk_status sk_acquire(SkDevice& D, hipStream_t s, size_t need, uint32_t nflags, SkWork*& out)
 {
@@ -1509,7 +1523,7 @@ mk_status sk_acquire(SkDevice& D, hipStream_t s, size_t need, uint32_t nflags, S
             pick = w.get();
     if (!pick)
         for (auto& w : D.pool)
-            if (w->ws_bytes >= need && w->nflags >= nflags && hipEventQuery(w->done) == hipSuccess) {
+            if (w->ws_bytes >= need && w->nflags >= nflags && sk_done(*w)) {
                 pick = w.get();
                 break;
             }
@@ -1532,7 +1546,10 @@ mk_status sk_acquire(SkDevice& D, hipStream_t s, size_t need, uint32_t nflags, S
                 pick = w.get();
         if (!pick)
             return fail(MK_ERR_UNSUPPORTED, "gemm: stream-K workspaces smaller than this launch needs");
-        MK_HIP(hipStreamWaitEvent(s, pick->done, 0));
+        if (hipStreamWaitEvent(s, pick->done, 0) != hipSuccess) { // its stream is gone: wait for the whole device
+            (void)hipGetLastError();
+            MK_HIP(hipDeviceSynchronize());
+        }
     }
     out = pick;
     return MK_OK;
@@ -1611,6 +1628,7 @@ mk_status launch(GemmP* p, uint32_t count, const GemmPlan& plan, hipStream_t s)
             MK_HIP(hipGetLastError());
             MK_HIP(hipEventRecord(W->done, s));
             W->last = s;
+            W->idle = false;
             W->used = ++D.launches;
             return MK_OK;
         }
@@ -1709,6 +1727,19 @@ mk_status prepare(const mk_gemm_args* a, GemmP& p, bool conv = false)
 }
 
 } // namespace gemm_detail
+
+void gemm_release_stream(const void* stream)
+{
+    using namespace gemm_detail;
+    std::lock_guard<std::mutex> lock(g_sk_mutex);
+    for (SkDevice& D : g_sk)
+        for (auto& w : D.pool)
+            if (w->last == stream && !w->idle) {
+                (void)hipEventSynchronize(w->done);
+                w->last = nullptr;
+                w->idle = true;
+            }
+}
 
 mk_status gemm_take_error(const void* stream, bool all)
 {

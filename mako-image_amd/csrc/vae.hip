@@ -626,8 +626,10 @@ struct mk_vae {
         for (Buf* b : {&x, &y, &t, &a, &sc, &qb, &kb, &vtb, &kf, &sb, &pb, &ob, &pj, &tok, &rgba, &probe_buf})
             if (b->p)
                 (void)hipFree(b->p);
-        if (stream)
+        if (stream) {
+            gemm_release_stream(stream);
             (void)hipStreamDestroy(stream);
+        }
     }
 
     mk_status alloc(size_t bytes, void** p)

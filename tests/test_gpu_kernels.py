@@ -526,6 +526,23 @@ def test_gemm_stream_k_on_two_streams_at_once(gpu, rng):
             M.call("mk_stream_destroy", st)
 
 
+def test_gemm_stream_k_after_its_stream_is_destroyed(gpu, rng):
+    # the workspace of a destroyed stream's launch goes to the next stream's: no launch reports the dead stream's event
+    P = _sk_problem(rng)
+    want = None
+    for _ in range(6):
+        h = C.c_void_p()
+        M.call("mk_stream_create", C.byref(h))
+        cs = _sk_launch(P, h.value)
+        M.call("mk_stream_destroy", h.value)
+        other = _sk_launch(P)
+        M.sync()
+        for got in (cs, other):
+            got = [fetch(c, (Mr, P["N"])) for c, Mr in zip(got, P["shapes"])]
+            want = want or got
+            assert all(np.array_equal(a, b) for a, b in zip(got, want))
+
+
 def test_gemm_stream_k_gave_up_wait_is_reported(gpu, rng):
     # a zero wait bound makes every owner of a split tile give up at once (the kernel still completes, from whatever
     # the partial slots hold); the next synchronisation reports it, once, and the default bound restores results
