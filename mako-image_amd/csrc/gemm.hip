@@ -353,35 +353,71 @@ __device__ inline void epi_heads(const GemmP& p, const float* st, int ld, int to
     const int which = nw0 / int(h.dim), head = (nw0 % int(h.dim)) / 128;
     const int64_t bh = int64_t(z) * h.heads + head;
     if (which == 2) {
-        float sc[2], bi[2];
-#pragma unroll
-        for (int dd = 0; dd < 2; ++dd) {
-            sc[dd] = p.wscale ? p.wscale[nw0 + 2 * lane + dd] : 1.0f;
-            bi[dd] = p.bias ? p.bias[nw0 + 2 * lane + dd] : 0.0f;
-        }
+        // a lane's two dims 2 lane, 2 lane + 1 of a token: one 8-byte LDS read
+        const int d = 2 * lane;
+        const float sc0 = p.wscale ? p.wscale[nw0 + d] : 1.0f, sc1 = p.wscale ? p.wscale[nw0 + d + 1] : 1.0f;
+        const float bi0 = p.bias ? p.bias[nw0 + d] : 0.0f, bi1 = p.bias ? p.bias[nw0 + d + 1] : 0.0f;
         const uint32_t k0 = h.row0 + tok0;
-        const bool full = k0 % 16 == 0 && tok0 + 32 <= int(p.M);
-#pragma unroll
-        for (int dd = 0; dd < 2; ++dd) {
-            const int d = 2 * lane + dd;
-            uint16_t* dst = h.vt + (bh * 128 + d) * int64_t(h.k_pad);
-            auto v = [&](int j) { return st[j * ld + d] * sc[dd] + bi[dd]; };
-            if (full) {
-#pragma unroll
-                for (int g = 0; g < 2; ++g) {
-                    // physical columns 16g + 0..15 hold keys 16g + {0..3, 8..11, 4..7, 12..15}
-                    const int j0 = 16 * g;
-                    *reinterpret_cast<u32x4*>(dst + k0 + j0) =
-                        u32x4{pack_x2(v(j0 + 0), v(j0 + 1), F16), pack_x2(v(j0 + 2), v(j0 + 3), F16),
-                              pack_x2(v(j0 + 8), v(j0 + 9), F16), pack_x2(v(j0 + 10), v(j0 + 11), F16)};
-                    *reinterpret_cast<u32x4*>(dst + k0 + j0 + 8) =
-                        u32x4{pack_x2(v(j0 + 4), v(j0 + 5), F16), pack_x2(v(j0 + 6), v(j0 + 7), F16),
-                              pack_x2(v(j0 + 12), v(j0 + 13), F16), pack_x2(v(j0 + 14), v(j0 + 15), F16)};
-                }
-            } else {
-                for (int t = 0; t < 32 && tok0 + t < int(p.M); ++t)
-                    dst[vt_col(k0 + t)] = F16 ? f2h_bits(v(t)) : f2bf_bits(v(t));
+        uint16_t* dst0 = h.vt + (bh * 128 + d) * int64_t(h.k_pad);
+        uint16_t* dst1 = dst0 + h.k_pad;
+        auto v = [&](int j) {
+            const f32x2v x = *reinterpret_cast<const f32x2v*>(st + j * ld + d);
+            return f32x2v{x[0] * sc0 + bi0, x[1] * sc1 + bi1};
+        };
+        // tokens t .. t + 3 as packed 16-bit pairs of each dim
+        auto four = [&](int t, u32x2& a, u32x2& b) {
+            const f32x2v x0 = v(t), x1 = v(t + 1), x2 = v(t + 2), x3 = v(t + 3);
+            a = u32x2{pack_x2(x0[0], x1[0], F16), pack_x2(x2[0], x3[0], F16)};
+            b = u32x2{pack_x2(x0[1], x1[1], F16), pack_x2(x2[1], x3[1], F16)};
+        };
+        if (tok0 + 32 > int(p.M)) {
+            for (int t = 0; t < 32 && tok0 + t < int(p.M); ++t) {
+                const f32x2v x = v(t);
+                const uint32_t col = vt_col(k0 + t);
+                dst0[col] = F16 ? f2h_bits(x[0]) : f2bf_bits(x[0]);
+                dst1[col] = F16 ? f2h_bits(x[1]) : f2bf_bits(x[1]);
             }
+        } else if (k0 % 16 == 0) {
+#pragma unroll
+            for (int g = 0; g < 2; ++g) {
+                // physical columns 16g + 0..15 hold keys 16g + {0..3, 8..11, 4..7, 12..15}
+                u32x2 a[4], b[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    four(16 * g + 4 * i, a[i], b[i]);
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    *reinterpret_cast<u32x4*>(dst0 + k0 + 16 * g + 8 * i) =
+                        u32x4{a[i][0], a[i][1], a[i + 2][0], a[i + 2][1]};
+                    *reinterpret_cast<u32x4*>(dst1 + k0 + 16 * g + 8 * i) =
+                        u32x4{b[i][0], b[i][1], b[i + 2][0], b[i + 2][1]};
+                }
+            }
+        } else {
+            // Keys that start inside a group of 16 (image rows behind a prompt of any length). The column order
+            // keeps aligned groups of 4 keys together, so the slice's whole groups go out as 8-byte stores and only
+            // the 4 keys of its two cut groups one by one (r at the front, 4 - r behind). Every key one by one was 64
+            // scattered 2-byte stores a lane: the grouped QKV launch of 2 x (3952 + 200) rows (fp8, image rows from
+            // key 200) took 622 us, 470 with the groups; 2 x (1024 + 131) rows in bf16 252 and 174.
+            const int r = int(-k0 & 3u); // keys before the first aligned group of 4
+#pragma unroll
+            for (int g = 0; g < 8; ++g)
+                if (g < 7 || r == 0) {
+                    u32x2 a, b;
+                    four(4 * g + r, a, b);
+                    const uint32_t col = vt_col(k0 + 4 * g + r);
+                    *reinterpret_cast<u32x2*>(dst0 + col) = a;
+                    *reinterpret_cast<u32x2*>(dst1 + col) = b;
+                }
+            if (r)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int t = e < r ? e : 28 + e;
+                    const f32x2v x = v(t);
+                    const uint32_t col = vt_col(k0 + t);
+                    dst0[col] = F16 ? f2h_bits(x[0]) : f2bf_bits(x[0]);
+                    dst1[col] = F16 ? f2h_bits(x[1]) : f2bf_bits(x[1]);
+                }
         }
         return;
     }

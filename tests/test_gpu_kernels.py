@@ -285,6 +285,28 @@ def test_gemm_heads_epilogue(gpu, rng, mode, row0, q_row0, k_scale, odt):
     assert not gq[:, :, :q_row0].any() and not gq[:, :, q_row0 + Mr:].any()
 
 
+# V^T of 128-dim heads behind a prompt of any length: every position of the first key in its group of 4 (whole groups
+# as 8-byte stores, the two cut ones key by key), whole 32-token slices and a cut last one, against the plain products
+@pytest.mark.parametrize("row0", [1, 2, 3, 4, 14, 16, 131])
+@pytest.mark.parametrize("Mr,odt", [(64, M.BF16), (97, M.F16)])
+def test_gemm_heads_vt_behind_any_prompt(gpu, rng, row0, Mr, odt):
+    H, K_, k_pad = 2, 64, 256
+    D = H * 128
+    A = rng.standard_normal((Mr, K_)).astype(np.float32)
+    W = R.bf16_round(rng.standard_normal((3 * D, K_)).astype(np.float32) * 0.1)
+    b = rng.standard_normal(3 * D).astype(np.float32)
+    Q, Kd, Vt = (dev(np.zeros(H * 256 * 128, np.uint16)) for _ in range(3))
+    ha = M.HeadsArgs(Q.p, Kd.p, Vt.p, H, 128, 256, k_pad, row0, 0, None, None, None, 0, 1e-6, 0.0, odt)
+    gemm(bdev(A), bdev(W), bias=dev(b), epi=M.EPI_HEADS, c_dtype=M.BF16, M_=(Mr, 3 * D, K_), lda=K_, heads=ha)
+    bits = fetch(Vt, (H, 128, k_pad), np.uint16)
+    got = M.f16_to_f32(bits) if odt == M.F16 else M.bf16_to_f32(bits)
+    want = R.gemm(A, W, b)[:, 2 * D:].reshape(Mr, H, 128).transpose(1, 2, 0)
+    cols = M.vt_col(np.arange(row0, row0 + Mr))
+    # one rounding to 11 (half) or 8 (bf16) bits of sums whose fp32 order differs
+    assert np.abs(got[:, :, cols] - want).max() <= 2 ** (-11 if odt == M.F16 else -8) * np.abs(want).max() + 1e-5
+    assert not np.delete(got, cols, 2).any()  # the keys before and behind stay zero
+
+
 # 64-dim heads (the SDXL form: half, no norm, no RoPE) on 128-channel tiles: q | k | v and Q alone, batch 2, row
 # counts that end inside a tile and inside a 16-key group; each value within one rounding (half or bf16) of the
 # oracle's GEMM, padding rows untouched (zero)
