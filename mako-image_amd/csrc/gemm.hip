@@ -16,6 +16,7 @@
 // along M.
 #include "common.hpp"
 
+#include <algorithm>
 #include <memory>
 #include <mutex>
 #include <type_traits>
@@ -1674,6 +1675,132 @@ mk_status launch(GemmP* p, uint32_t count, const GemmPlan& plan, hipStream_t s)
     return MK_OK;
 }
 
+// C[M][64] = A W^T + bias with 64 output channels (the output head). On 256 x 64 tiles the head of 8192 rows is 32
+// workgroups of 48 k steps each; here a workgroup takes 32 tokens, and its 4 waves a quarter of K each: every wave
+// stages its own k steps (96 rows of 64 values: 64 of W, 32 of A) in its own LDS by direct loads, three k steps ahead,
+// without a barrier, and the waves' sums meet in LDS once, added in wave order. (The fragments straight from global
+// memory touch 32 lines a load, each line four times: 27 us at 256 rows, 31 at 8192.) Bound by load latency up to
+// 2048 rows and by the 64 channels' weights every workgroup reads through L2 beyond. Isolated launches, K = 3072: 256
+// rows 36.6 -> 7.6 us, 2048 37.4 -> 9.9, 8192 37.3 -> 12.8 (3.9 TB/s of A), 16384 60 -> 32.
+template <bool kF16> __global__ __launch_bounds__(256, 1) void gemm_n64_kernel(GemmP p)
+{
+    constexpr int NW = 4, LD = 64 + 4, ROWS = 64 + 32, NL = ROWS / 8, WE = ROWS * 64; // loads, elements a wave's step
+    // a stage is an object of its own, so the reads of one do not wait for the loads into another
+    __shared__ __attribute__((aligned(16))) uint16_t s0[NW * WE], s1[NW * WE], s2[NW * WE];
+    auto stage = [&](int i) { return i == 0 ? s0 : i == 1 ? s1 : s2; };
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r32 = lane & 31, hk = lane >> 5;
+    const uint32_t z = blockIdx.x / p.tiles_m, tm = blockIdx.x - z * p.tiles_m;
+    const int m0 = int(tm) * 32, kt = int(p.K) / BK, kb = kt * wave / NW, ke = kt * (wave + 1) / NW;
+    const BufRes rsW = buf_res(p.w, uint32_t(64u * p.K * 2));
+    const BufRes rsA = buf_res(p.a + int64_t(z) * p.sa + int64_t(m0) * p.lda,
+                               uint32_t(((min(int(p.M) - m0, 32) - 1) * int64_t(p.lda) + p.K) * 2));
+    uint32_t off[NL];
+#pragma unroll
+    for (int i = 0; i < NL; ++i) { // rows past M read the last row
+        const int P = i * 64 + lane, row = P >> 3, kc = swz_chunk(row, P & 7);
+        off[i] = i < 8 ? uint32_t(row * int(p.K) + kc * 8) * 2
+                       : uint32_t(min(row - 64, int(p.M) - 1 - m0) * int(p.lda) + kc * 8) * 2;
+    }
+    auto issue = [&](auto st_c, int k) { // past the end: the last step again (unused)
+        constexpr int st = decltype(st_c)::value;
+        const uint32_t o = uint32_t(min(k, kt - 1) * BK * 2);
+#pragma unroll
+        for (int i = 0; i < NL; ++i)
+            buf_load_lds16(i < 8 ? rsW : rsA, (lds_void*)&stage(st)[wave * WE + i * 512], off[i], o);
+    };
+    f32x16 acc[2] = {f32x16{}, f32x16{}};
+    auto step = [&](auto st_c, int k) {
+        constexpr int st = decltype(st_c)::value;
+        __builtin_amdgcn_s_waitcnt(waitcnt_bits(2 * NL, 0)); // step k landed, the next two may be in flight
+        const uint16_t* w = stage(st) + wave * WE;
+        bf16x8 f[4][3];
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+                f[ks][j] = *reinterpret_cast<const bf16x8*>(&w[swz(32 * j + r32, ks * 2 + hk)]);
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+            for (int cb = 0; cb < 2; ++cb) {
+                if constexpr (kF16)
+                    acc[cb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8v, f[ks][cb]),
+                                                                     __builtin_bit_cast(f16x8v, f[ks][2]), acc[cb], 0,
+                                                                     0, 0);
+                else
+                    acc[cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[ks][cb], f[ks][2], acc[cb], 0, 0, 0);
+            }
+        __builtin_amdgcn_sched_barrier(0); // the reads are done (the products took them) before the stage is refilled
+        issue(st_c, k + 3);
+    };
+    using S0 = std::integral_constant<int, 0>;
+    using S1 = std::integral_constant<int, 1>;
+    using S2 = std::integral_constant<int, 2>;
+    issue(S0{}, kb);
+    issue(S1{}, kb + 1);
+    issue(S2{}, kb + 2);
+    int k = kb;
+    for (; k + 2 < ke; k += 3) {
+        step(S0{}, k);
+        step(S1{}, k + 1);
+        step(S2{}, k + 2);
+    }
+    if (k < ke)
+        step(S0{}, k);
+    if (k + 1 < ke)
+        step(S1{}, k + 1);
+    __builtin_amdgcn_s_waitcnt(0); // the last (unused) loads land before the LDS is reused
+    __syncthreads();
+    // a lane holds channels 32 cb + 8 i + 4 hk .. + 3 of token r32
+    static_assert(NW * 32 * LD * 4 <= NW * WE * 2, "the sums fit a stage");
+    float* part = reinterpret_cast<float*>(s0);
+#pragma unroll
+    for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            *reinterpret_cast<f32x4*>(part + (wave * 32 + r32) * LD + 32 * cb + 8 * i + 4 * hk) =
+                f32x4{acc[cb][4 * i], acc[cb][4 * i + 1], acc[cb][4 * i + 2], acc[cb][4 * i + 3]};
+    __syncthreads();
+    const int ch = 4 * (threadIdx.x & 15);
+    const f32x4 bias = p.bias ? *reinterpret_cast<const f32x4*>(p.bias + ch) : f32x4{0, 0, 0, 0};
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int row = 16 * h + int(threadIdx.x >> 4), t = m0 + row;
+        f32x4 v = *reinterpret_cast<const f32x4*>(part + row * LD + ch);
+#pragma unroll
+        for (int w = 1; w < NW; ++w) {
+            const f32x4 u = *reinterpret_cast<const f32x4*>(part + (w * 32 + row) * LD + ch);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                v[e] += u[e];
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            v[e] += bias[e];
+        if (t >= int(p.M))
+            continue;
+        const int64_t o = int64_t(z) * p.sc + int64_t(t) * p.ldc + ch;
+        if (!p.c_bf16)
+            *reinterpret_cast<f32x4*>(static_cast<float*>(p.c) + o) = v;
+        else
+            *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(p.c) + o) =
+                p.c_f16 ? u32x2{pack_f16x2(v[0], v[1]), pack_f16x2(v[2], v[3])}
+                        : u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+    }
+}
+
+mk_status launch_n64(GemmP& p, bool f16, hipStream_t s)
+{
+    p.tiles_m = cdiv(p.M, 32);
+    if (f16)
+        gemm_n64_kernel<true><<<p.tiles_m * p.batch, 256, 0, s>>>(p);
+    else
+        gemm_n64_kernel<false><<<p.tiles_m * p.batch, 256, 0, s>>>(p);
+    MK_HIP(hipGetLastError());
+    return MK_OK;
+}
+
 // The epilogue kind of an mk_epilogue.
 int epi_kind(uint32_t e)
 {
@@ -1904,6 +2031,13 @@ extern "C" mk_status mk_gemm_grouped(const mk_gemm_args* a, uint32_t count, void
     if (ek == EK_HEADS && !((bn == 256 && p[0].hp.hd == 128) || (bn == 128 && p[0].hp.hd == 64)))
         return fail(MK_ERR_UNSUPPORTED, "gemm: heads epilogue tile width does not match the head dim");
     hipStream_t s = static_cast<hipStream_t>(stream);
+    // 64 channels stored: gemm_n64_kernel up to as many rounds of its workgroups as it wins (K = 3072: 32768 rows, 4
+    // rounds, 61 us against 67 on 256 x 64 tiles, 65536 rows 118 against 88; K = 384: 4096 rows, half a round, 4.5
+    // against 6.7, 30000 rows, 3.7 rounds, 15.1 against 9.7)
+    const uint64_t rounds64 = std::min<uint64_t>(4, std::max<uint64_t>(1, a[0].K / 768));
+    if (n == 1 && p[0].N == 64 && ek == EK_STORE && !f8 && !p[0].wscale &&
+        uint64_t(cdiv(p[0].M, 32)) * p[0].batch <= rounds64 * uint64_t(cus > 0 ? cus : 1))
+        return launch_n64(p[0], a[0].w_dtype == MK_F16, s);
     mk_status e;
     // 4-wave 128-channel tiles (128 x 128, or 256 x 128 with bn 128) of epilogue kind E: deep-staged (EK_DEEP) when
     // the launch has at most one tile a CU, so each workgroup runs alone on its CU

@@ -285,6 +285,31 @@ def test_gemm_heads_epilogue(gpu, rng, mode, row0, q_row0, k_scale, odt):
     assert not gq[:, :, :q_row0].any() and not gq[:, :, q_row0 + Mr:].any()
 
 
+# 64 output channels take a kernel of their own: row counts that end inside its 32-token tiles, K of fewer k steps than
+# its 4 waves, of whole and of cut rounds of its 3 stages, strides, batch items and each output type
+@pytest.mark.parametrize("Mr,K", [(1, 64), (31, 192), (33, 832), (64, 768), (300, 3072), (8200, 1536)])
+@pytest.mark.parametrize("wdt,cdt", [(M.BF16, M.F32), (M.BF16, M.BF16), (M.F16, M.F16)])
+def test_gemm_64_channels(gpu, rng, Mr, K, wdt, cdt):
+    B, N, lda, ldc = 2, 64, K + 64, 72
+    rnd, bits = (R.f16_round, M.f16_bits) if wdt == M.F16 else (R.bf16_round, M.bf16_bits)
+    A = rnd(rng.standard_normal((B, Mr, lda)).astype(np.float32))
+    W = rnd(rng.standard_normal((N, K)).astype(np.float32) * 0.05)
+    b = rng.standard_normal(N).astype(np.float32)
+    esz = 4 if cdt == M.F32 else 2
+    out = dev(np.full(B * (Mr + 1) * ldc * esz, 0x11, np.uint8))
+    gemm(dev(bits(A)), dev(bits(W)), bias=dev(b), c=out, c_dtype=cdt, M_=(Mr, N, K), batch=B, lda=lda, ldc=ldc,
+         sa=Mr * lda, sc=(Mr + 1) * ldc, w_dtype=wdt)
+    raw = fetch(out, (B, Mr + 1, ldc), np.float32 if cdt == M.F32 else np.uint16)
+    got = raw if cdt == M.F32 else (M.f16_to_f32 if cdt == M.F16 else M.bf16_to_f32)(raw)
+    rows = np.unique(np.r_[0, Mr - 1, rng.choice(Mr, min(Mr, 64), replace=False)])
+    for i in range(B):
+        want = A[i, rows, :K].astype(np.float64) @ W.T.astype(np.float64) + b
+        # fp32 sums of K products, then one rounding to the output type
+        tol = 1e-5 + (0 if cdt == M.F32 else 2 ** -11 if cdt == M.F16 else 2 ** -8)
+        assert np.abs(got[i, rows, :N] - want).max() <= tol * np.abs(want).max()
+        assert (raw[i].view(np.uint8)[Mr] == 0x11).all() and (raw[i][:, N:].copy().view(np.uint8) == 0x11).all()
+
+
 # V^T of 128-dim heads behind a prompt of any length: every position of the first key in its group of 4 (whole groups
 # as 8-byte stores, the two cut ones key by key), whole 32-token slices and a cut last one, against the plain products
 @pytest.mark.parametrize("row0", [1, 2, 3, 4, 14, 16, 131])
