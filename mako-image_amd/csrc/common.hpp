@@ -55,6 +55,7 @@ struct GemmPlan {
     uint64_t tiles;  // tiles of the launch
     bool sk;         // stream-K: whole waves round robin, the last partial wave split by k steps
     uint64_t dp;     // tiles done whole (stream-K)
+    int splits;      // workgroups a 128 x 128 tile's k steps are split over (0 or 1: whole tiles of bm x bn)
     double cost;     // estimated duration in units of one k step of a 256 x 256 tile
 };
 // The plan of a launch of n grouped problems (equal N, K, weight type, epilogue kind) on `cus` compute units;

@@ -746,11 +746,11 @@ __device__ inline void epi_norm_silu(const GemmP& p, const float* st, int ld, in
 
 // One tile's k steps [kb, ke): the pipelined main loop, then either the partial published to stream-K slot
 // `publish`, or the partials of the tile's other ranges (virtual indices fix_lo .. fix_hi except `self`, tail tile
-// tt) added in index order, and the epilogue.
+// tt) added in index order, and the epilogue (C at c_off elements further on).
 template <int BM, int BN, bool kF8, int EK, int NW>
 __device__ __forceinline__ void gemm_tile(const GemmP& p, uint32_t z, uint32_t tm, uint32_t tn, int kb, int ke,
                                           uint16_t* smem, const SkP* sk, int publish, int fix_lo = 0,
-                                          int fix_hi = -1, int self = -1, uint64_t tt = 0)
+                                          int fix_hi = -1, int self = -1, uint64_t tt = 0, int64_t c_off = 0)
 {
     static_assert(((EK & 7) != EK_HEADS && (EK & 7) != EK_GLU) || !(EK & EK_CONV),
                   "a convolution has no heads or GLU epilogue");
@@ -1264,7 +1264,7 @@ __device__ __forceinline__ void gemm_tile(const GemmP& p, uint32_t z, uint32_t t
     // order, so the slices need no barrier (a __syncthreads() here would also wait for every global store in flight:
     // its release fence waits for vmcnt 0) ----
     float* st = reinterpret_cast<float*>(smem) + wave * 32 * LDW;
-    const int64_t zc = int64_t(z) * p.sc;
+    const int64_t zc = int64_t(z) * p.sc + c_off;
     // the wave's 32-token slice s (token blocks s for 32 x 32 x 16, 2 s and 2 s + 1 for 16 x 16 x 32) into st
     auto stage = [&](int s) {
 #pragma unroll
@@ -1451,6 +1451,100 @@ __global__ __launch_bounds__(64 * NW, BM == 128 && !(EK & EK_DEEP) ? 2 : 1) __at
     gemm_tile<BM, BN, kF8, EK, NW>(p, z, tm, tn, 0, int(p.K) / BK, smem, nullptr, -1);
 }
 
+// Split-K for launches of few tiles (a prompt's rows, a small image): `splits` workgroups share a tile's k steps and
+// store their fp32 partial tiles, unscaled, one slab of all rows a split; gemm_reduce_kernel then adds the slabs in
+// order and runs the epilogue. G holds the partials' C (the slab; its row stride N, no scale, bias or gate).
+template <int BM, int BN, bool kF8, int EK, int NW>
+__global__ __launch_bounds__(64 * NW, BM == 128 && !(EK & EK_DEEP) ? 2 : 1) __attribute__((amdgpu_waves_per_eu(
+    gemm_waves_per_eu<BM, NW, EK>(), gemm_waves_per_eu<BM, NW, EK>()))) void gemm_split_kernel(GemmG G, uint32_t splits,
+                                                                                            uint32_t tiles,
+                                                                                            uint64_t slab)
+{
+    __shared__ __attribute__((aligned(16))) uint16_t smem[gemm_smem<BM, BN, NW, (EK & EK_DEEP) != 0>() / 2];
+    // split-major: an XCD's run of workgroups shares its splits' columns of A
+    const uint32_t i = xcd_order(blockIdx.x, gridDim.x), s = i / tiles;
+    uint32_t z, tm, tn;
+    const GemmP& p = locate(G, i - s * tiles, z, tm, tn);
+    const uint32_t kt = p.K / BK;
+    gemm_tile<BM, BN, kF8, EK, NW>(p, z, tm, tn, int(kt * s / splits), int(kt * (s + 1) / splits), smem, nullptr, -1, 0,
+                                   -1, -1, 0, int64_t(s * slab));
+}
+
+// The sums of a split launch's slabs (`slab` floats apart, rows of N; problem 1's rows after problem 0's) through the
+// epilogue: 4 channels of a row a thread, the slabs added in order.
+template <int EK> __global__ __launch_bounds__(256) void gemm_reduce_kernel(GemmG G, const float* ws, uint32_t splits,
+                                                                            uint64_t slab, uint32_t items)
+{
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= items)
+        return;
+    constexpr bool kGlu = EK == EK_GLU;
+    const uint32_t N = G.g[0].N, nc = kGlu ? N / 8 : N / 4; // channel groups a row
+    const uint32_t row = i / nc, ch = 4 * (i - row * nc), rows0 = G.g[0].M * G.g[0].batch;
+    const GemmP& p = G.g[row >= rows0];
+    const uint32_t r = row >= rows0 ? row - rows0 : row, z = r / p.M, t = r - z * p.M;
+    const float* src = ws + uint64_t(row) * N + ch;
+    auto sum = [&](uint32_t c) {
+        f32x4 v{0, 0, 0, 0};
+        for (uint32_t s0 = 0; s0 < splits; s0 += 4) { // four slabs' loads in flight
+            f32x4 x[4];
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j)
+                x[j] = *reinterpret_cast<const f32x4*>(src + c + min(s0 + j, splits - 1) * slab);
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j)
+                if (s0 + j < splits)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        v[e] += x[j][e];
+        }
+        const uint32_t n = ch + c;
+        const f32x4 sc = p.wscale ? *reinterpret_cast<const f32x4*>(p.wscale + n) : f32x4{1, 1, 1, 1};
+        const f32x4 bi = p.bias ? *reinterpret_cast<const f32x4*>(p.bias + n) : f32x4{0, 0, 0, 0};
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            v[e] = v[e] * sc[e] + bi[e];
+        return v;
+    };
+    f32x4 v = sum(0);
+    const int64_t o = int64_t(z) * p.sc + int64_t(t) * p.ldc + ch;
+    if constexpr (EK == EK_RMW) {
+        float* c = static_cast<float*>(p.c) + o;
+        f32x4 x = *reinterpret_cast<const f32x4*>(c);
+        f32x4 g{1, 1, 1, 1};
+        if (p.epi != MK_EPI_ADD) {
+            g = *reinterpret_cast<const f32x4*>(p.gate + (t % p.seg_rows < p.split ? p.gate_alt : 0) + ch);
+            if (p.epi == MK_EPI_GATE_TANH)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    g[e] = tanh_f(g[e]);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            x[e] += g[e] * v[e];
+        *reinterpret_cast<f32x4*>(c) = x;
+        return;
+    }
+    if constexpr (kGlu) {
+        const f32x4 g = sum(p.glu_f);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            v[e] = p.epi == MK_EPI_PAIR_SUM ? v[e] + g[e]
+                   : p.epi == MK_EPI_SWIGLU ? silu_f(v[e]) * g[e]
+                                            : v[e] * (0.5f * g[e] * (1.0f + erf_fit(g[e] * 0.70710678f)));
+    }
+    if constexpr (EK == EK_ACT)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            v[e] = p.epi == MK_EPI_GELU_TANH ? gelu_tanh_f(v[e]) : silu_f(v[e]);
+    if (!p.c_bf16)
+        *reinterpret_cast<f32x4*>(static_cast<float*>(p.c) + o) = v;
+    else
+        *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(p.c) + o) =
+            p.c_f16 ? u32x2{pack_f16x2(v[0], v[1]), pack_f16x2(v[2], v[3])}
+                    : u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+}
+
 // Persistent stream-K: a grid of one workgroup a CU takes the first sk.dp tiles whole (round robin), then splits
 // the rest's k steps evenly into one range a workgroup. A tile split over several ranges is finished by the one
 // held by the highest workgroup: it adds the partials the others publish. Waits thus only ever point at workgroups
@@ -1615,6 +1709,139 @@ mk_status sk_check(SkDevice& D, hipStream_t s, bool all)
     for (auto& e : D.errs)
         if ((all || e.first == s) && __atomic_exchange_n(e.second, 0u, __ATOMIC_RELAXED))
             return fail(MK_ERR_DEVICE, "gemm: a stream-K launch gave up waiting for a partial tile; its output is wrong");
+    return MK_OK;
+}
+
+// Slabs of split-K launches: up to kSplitPool buffers of kSplitBytes a device, one a stream, so a stream's launches
+// follow each other on its own buffer and streams never share one. A stream beyond the pool takes the least recently
+// used buffer over after a device-wide wait; a destroyed stream's is given back by gemm_release_stream. (32 MB of slabs
+// stay in the memory-side cache between the two kernels.) Locked with g_sk_mutex over both launches.
+constexpr size_t kSplitBytes = size_t(32) << 20, kSplitPool = 8;
+struct SplitWork {
+    float* ws = nullptr;
+    hipStream_t owner = nullptr;
+    bool owned = false;
+    uint64_t used = 0;
+};
+struct SplitDevice {
+    uint64_t launches = 0;
+    std::vector<SplitWork> pool;
+};
+SplitDevice g_split[kMaxDevices];
+
+// The buffer of stream s (g_sk_mutex held); null when it cannot be had now (another stream is being captured).
+float* split_acquire(SplitDevice& D, hipStream_t s)
+{
+    SplitWork* pick = nullptr;
+    for (auto& w : D.pool)
+        if (w.owned && w.owner == s)
+            pick = &w;
+    if (!pick)
+        for (auto& w : D.pool)
+            if (!w.owned)
+                pick = &w;
+    if (!pick && D.pool.size() < kSplitPool) {
+        void* p = nullptr;
+        if (hipMalloc(&p, kSplitBytes) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        D.pool.push_back(SplitWork{static_cast<float*>(p)});
+        pick = &D.pool.back();
+    }
+    if (!pick) {
+        if (hipDeviceSynchronize() != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        for (auto& w : D.pool)
+            if (!pick || w.used < pick->used)
+                pick = &w;
+    }
+    pick->owner = s;
+    pick->owned = true;
+    pick->used = ++D.launches;
+    return pick->ws;
+}
+
+template <int EK> void launch_reduce(const GemmG& G, const float* ws, uint32_t splits, uint64_t slab, uint32_t rows,
+                                     hipStream_t s)
+{
+    const uint32_t items = rows * (EK == EK_GLU ? G.g[0].N / 8 : G.g[0].N / 4);
+    gemm_reduce_kernel<EK><<<cdiv(items, 256), 256, 0, s>>>(G, ws, splits, slab, items);
+}
+
+// A split launch of `plan.splits` k ranges a 128 x 128 tile; `done` is left false when the stream is being captured or
+// no slab buffer can be had (a captured launch must not own memory another launch may use): the caller then launches
+// whole tiles.
+mk_status launch_split(GemmP* p, uint32_t count, const GemmPlan& plan, int ek, bool f8, bool f16, uint32_t cus,
+                       hipStream_t s, bool& done)
+{
+    done = false;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
+        (void)hipGetLastError();
+        return MK_OK;
+    }
+    if (cap != hipStreamCaptureStatusNone)
+        return MK_OK;
+    int dev = 0;
+    MK_HIP(hipGetDevice(&dev));
+    if (dev < 0 || dev >= kMaxDevices)
+        return fail(MK_ERR_DEVICE, "gemm: device index out of range");
+    GemmG G{}, P{}; // the epilogue's problems, the partials'
+    uint32_t tiles = 0, rows = 0;
+    for (uint32_t i = 0; i < count; ++i) {
+        p[i].tiles_m = cdiv(p[i].M, 128);
+        p[i].tiles_n = p[i].N / 128;
+        G.g[i] = P.g[i] = p[i];
+        rows += p[i].M * p[i].batch;
+        tiles += p[i].tiles_m * p[i].tiles_n * p[i].batch;
+    }
+    const uint32_t N = p[0].N, splits = uint32_t(plan.splits);
+    const uint64_t slab = uint64_t(rows) * N;
+    if (slab * splits * 4 > kSplitBytes)
+        return MK_OK;
+    std::lock_guard<std::mutex> lock(g_sk_mutex);
+    float* ws = split_acquire(g_split[dev], s);
+    if (!ws)
+        return MK_OK;
+    uint32_t r0 = 0;
+    for (uint32_t i = 0; i < count; ++i) {
+        GemmP& q = P.g[i];
+        q.c = ws + uint64_t(r0) * N;
+        q.ldc = N;
+        q.sc = int64_t(q.M) * N;
+        q.wscale = nullptr;
+        q.bias = q.gate = nullptr;
+        q.epi = MK_EPI_STORE;
+        q.c_bf16 = q.c_f16 = q.glu_f = 0;
+        r0 += q.M * q.batch;
+    }
+    P.tiles0 = count > 1 ? p[0].tiles_m * p[0].tiles_n * p[0].batch : tiles;
+    const uint32_t wgs = tiles * splits;
+    constexpr int H = EK_STORE | EK_F16;
+    if (f8)
+        gemm_split_kernel<128, 128, true, EK_STORE, 4><<<wgs, 256, 0, s>>>(P, splits, tiles, slab);
+    else if (f16 && wgs <= cus)
+        gemm_split_kernel<128, 128, false, H | EK_DEEP, 4><<<wgs, 256, 0, s>>>(P, splits, tiles, slab);
+    else if (f16)
+        gemm_split_kernel<128, 128, false, H, 4><<<wgs, 256, 0, s>>>(P, splits, tiles, slab);
+    else if (wgs <= cus)
+        gemm_split_kernel<128, 128, false, EK_STORE | EK_DEEP, 4><<<wgs, 256, 0, s>>>(P, splits, tiles, slab);
+    else
+        gemm_split_kernel<128, 128, false, EK_STORE, 4><<<wgs, 256, 0, s>>>(P, splits, tiles, slab);
+    MK_HIP(hipGetLastError());
+    if (ek == EK_STORE)
+        launch_reduce<EK_STORE>(G, ws, splits, slab, rows, s);
+    else if (ek == EK_ACT)
+        launch_reduce<EK_ACT>(G, ws, splits, slab, rows, s);
+    else if (ek == EK_GLU)
+        launch_reduce<EK_GLU>(G, ws, splits, slab, rows, s);
+    else
+        launch_reduce<EK_RMW>(G, ws, splits, slab, rows, s);
+    MK_HIP(hipGetLastError());
+    done = true;
     return MK_OK;
 }
 
@@ -1902,6 +2129,12 @@ void gemm_release_stream(const void* stream)
                 w->last = nullptr;
                 w->idle = true;
             }
+    for (SplitDevice& D : g_split)
+        for (auto& w : D.pool)
+            if (w.owned && w.owner == stream) {
+                (void)hipStreamSynchronize(w.owner);
+                w.owned = false;
+            }
 }
 
 mk_status gemm_take_error(const void* stream, bool all)
@@ -1984,6 +2217,30 @@ GemmPlan gemm_plan(const mk_gemm_args* a, uint32_t n, uint32_t cus, bool conv)
         consider(128, 128, 0.67);
     if (best.cost < 0) // N not a multiple of 128 with an activation or GLU: the dispatch rejects it
         consider(256, 64, 0.62);
+    // Few rows and long K: split each 128 x 128 tile's k steps over S workgroups (gemm_split_kernel), at most one a CU.
+    // In us, a k step takes 0.42, a split adds 0.3 and its slab's write and read at 2.5 TB/s, the reduce launch 3; S is
+    // the one with the least sum, 1 included. Measured (isolated launches, whole tiles -> the rule's S; the best S of a
+    // sweep over 2-16 is within 10%): 77 x 3072 x 12288 98 -> 25 us (S 10), 320 x 3072 x 12288 101 -> 48 (3), fp8 128 x
+    // 3072 x 12288 120 -> 24 (10), 64 x 3072 x 3584 19.9 -> 12.5 (6), 77 x 12288 x 3072 33 -> 28 (2), f16 512 x 1280 x
+    // 5120 34 -> 20 (5); 512 x 1280 x 1280 stays whole (13.6 against 14.0). More than 512 rows stay whole too, so that
+    // the parts of an image's rows launched apart get the bits of one launch.
+    uint64_t rows = 0;
+    for (uint32_t i = 0; i < n; ++i)
+        rows += uint64_t(a[i].M) * a[i].batch;
+    if (!conv && N % 128 == 0 && rows <= 512) {
+        const uint64_t cap = cus / std::max<uint64_t>(1, tiles_of(128, 128));
+        const double slab = double(rows) * N * 4, whole = 0.42 * double(kt);
+        double least = whole;
+        for (uint64_t sp = 2; sp <= cap && sp <= kt && double(sp) * slab <= double(gemm_detail::kSplitBytes); ++sp) {
+            const double t = whole / double(sp) + 3.0 + double(sp) * (0.3 + slab / 2.5e6);
+            if (t < least) {
+                least = t;
+                best.splits = int(sp);
+            }
+        }
+        if (best.splits > 1)
+            best.cost = std::min(best.cost, least / 1.6); // a 256 x 256 k step takes 1.6 us
+    }
     return best;
 }
 
@@ -2038,6 +2295,12 @@ extern "C" mk_status mk_gemm_grouped(const mk_gemm_args* a, uint32_t count, void
     if (n == 1 && p[0].N == 64 && ek == EK_STORE && !f8 && !p[0].wscale &&
         uint64_t(cdiv(p[0].M, 32)) * p[0].batch <= rounds64 * uint64_t(cus > 0 ? cus : 1))
         return launch_n64(p[0], a[0].w_dtype == MK_F16, s);
+    if (plan.splits > 1 && !(ek == EK_ACT && a[0].w_dtype == MK_F16)) {
+        bool done = false;
+        MK_TRY(launch_split(p, n, plan, ek, f8, a[0].w_dtype == MK_F16, uint32_t(cus > 0 ? cus : 1), s, done));
+        if (done)
+            return MK_OK;
+    }
     mk_status e;
     // 4-wave 128-channel tiles (128 x 128, or 256 x 128 with bn 128) of epilogue kind E: deep-staged (EK_DEEP) when
     // the launch has at most one tile a CU, so each workgroup runs alone on its CU

@@ -285,6 +285,88 @@ def test_gemm_heads_epilogue(gpu, rng, mode, row0, q_row0, k_scale, odt):
     assert not gq[:, :, :q_row0].any() and not gq[:, :, q_row0 + Mr:].any()
 
 
+# Few rows and long K: the k steps split over workgroups, the slabs added and put through the epilogue by a second
+# kernel. One row, rows that end inside a tile, the most rows that split, uneven k ranges (K of 9 to 192 k steps), every
+# epilogue, weight type and output type, against the oracle's product; a second launch repeats the bits.
+@pytest.mark.parametrize("Mr,N,K", [(1, 128, 2048), (77, 384, 6144), (512, 256, 1600), (130, 128, 12288)])
+@pytest.mark.parametrize("epi,wdt", [(M.EPI_STORE, M.BF16), (M.EPI_STORE, M.FP8), (M.EPI_STORE, M.F16),
+                                     (M.EPI_GATE_TANH, M.BF16), (M.EPI_GATE_ADD, M.FP8), (M.EPI_ADD, M.F16),
+                                     (M.EPI_GELU_TANH, M.BF16), (M.EPI_SILU, M.FP8), (M.EPI_SWIGLU, M.BF16),
+                                     (M.EPI_GEGLU, M.F16), (M.EPI_PAIR_SUM, M.F16)])
+def test_gemm_split_k(gpu, rng, Mr, N, K, epi, wdt):
+    rnd, bits = (R.f16_round, M.f16_bits) if wdt == M.F16 else (R.bf16_round, M.bf16_bits)
+    A = rnd(rng.standard_normal((Mr, K)).astype(np.float32))
+    Wf = rng.standard_normal((N, K)).astype(np.float32) * 0.03
+    scale = None
+    if wdt == M.FP8:
+        codes = rng.integers(0, 127, (N, K)).astype(np.uint8) | (rng.integers(0, 2, (N, K)) << 7).astype(np.uint8)
+        scale = rng.uniform(0.5, 1.5, N).astype(np.float32) * 1e-3
+        Wq, Wd = R.e4m3_table()[codes] * scale[:, None], dev(codes)
+    else:
+        Wq = rnd(Wf)
+        Wd = dev(bits(Wq))
+    b = rng.standard_normal(N).astype(np.float32) * 0.3
+    glu = epi in (M.EPI_SWIGLU, M.EPI_GEGLU, M.EPI_PAIR_SUM)
+    F = N // 2 if glu else N
+    resid = epi in (M.EPI_GATE_TANH, M.EPI_GATE_ADD, M.EPI_ADD)
+    out16 = epi in (M.EPI_GELU_TANH, M.EPI_SILU, M.EPI_SWIGLU, M.EPI_GEGLU)
+    odt = (M.F16 if wdt == M.F16 else M.BF16) if out16 else M.F32
+    gates = rng.standard_normal((2, N)).astype(np.float32)
+    X = rng.standard_normal((Mr, F)).astype(np.float32)
+    y = A.astype(np.float64) @ Wq.T.astype(np.float64) + b
+    gate = np.where(np.arange(Mr)[:, None] < 37, gates[1], gates[0])
+    want = {M.EPI_STORE: lambda: y, M.EPI_ADD: lambda: X + y, M.EPI_GATE_ADD: lambda: X + gate * y,
+            M.EPI_GATE_TANH: lambda: X + np.tanh(gate) * y, M.EPI_GELU_TANH: lambda: R.gelu_tanh(y.astype(np.float32)),
+            M.EPI_SILU: lambda: y / (1 + np.exp(-y)), M.EPI_SWIGLU: lambda: y[:, :F] / (1 + np.exp(-y[:, :F])) * y[:, F:],
+            M.EPI_GEGLU: lambda: R.geglu(y.astype(np.float32)), M.EPI_PAIR_SUM: lambda: y[:, :F] + y[:, F:]}[epi]()
+    Ad, bd, gd, sd = dev(bits(A)), dev(b), dev(gates), None if scale is None else dev(scale)
+    outs = []
+    for _ in range(2):
+        out = dev(X if resid else np.zeros((Mr, F), np.uint16 if out16 else np.float32))
+        gemm(Ad, Wd, bias=bd, wscale=sd, c=out, c_dtype=odt, epi=epi, M_=(Mr, N, K), lda=K, ldc=F, w_dtype=wdt,
+             gate=gd if epi in (M.EPI_GATE_TANH, M.EPI_GATE_ADD) else None, gate_alt=N, split=37, seg=Mr)
+        raw = fetch(out, (Mr, F), np.uint16 if out16 else np.float32)
+        outs.append((M.f16_to_f32 if odt == M.F16 else M.bf16_to_f32)(raw) if out16 else raw)
+    assert np.array_equal(outs[0], outs[1])
+    # fp32 sums (relative to the largest product sum) and, for 16-bit outputs, one rounding
+    tol = 1e-5 + (0 if not out16 else 2 ** -11 if odt == M.F16 else 2 ** -8)
+    assert np.abs(outs[0] - want).max() <= tol * max(np.abs(want).max(), np.abs(y).max())
+
+
+def test_gemm_split_k_grouped_on_many_streams(gpu, rng):
+    # two problems a launch on more streams than there are slab buffers, all in flight together: every launch has the
+    # bits of the same one run alone
+    N, K, shapes = 256, 4096, (200, 40)
+    A = [bdev(rng.standard_normal((m, K)).astype(np.float32)) for m in shapes]
+    W, b = bdev(rng.standard_normal((N, K)).astype(np.float32) * 0.03), dev(rng.standard_normal(N).astype(np.float32))
+
+    def launch(stream):
+        cs = [dev(np.zeros((m, N), np.float32)) for m in shapes]
+        arr = (M.GemmArgs * 2)(*[gemm_args(a, W, bias=b, c=c, M_=(m, N, K), lda=K, ldc=N)
+                                 for a, c, m in zip(A, cs, shapes)])
+        _live.append(arr)
+        M.call("mk_gemm_grouped", C.cast(arr, C.c_void_p), 2, stream)
+        return cs
+
+    alone = launch(None)
+    M.sync()
+    want = [fetch(c, (m, N)) for c, m in zip(alone, shapes)]
+    streams = []
+    for _ in range(11):
+        h = C.c_void_p()
+        M.call("mk_stream_create", C.byref(h))
+        streams.append(h.value)
+    runs = [launch(s) for _ in range(2) for s in streams]
+    M.sync()
+    for s in streams:
+        M.call("mk_stream_destroy", s)
+    runs.append(launch(None))
+    M.sync()
+    for cs in runs:
+        for c, m, w in zip(cs, shapes, want):
+            assert np.array_equal(fetch(c, (m, N)), w)
+
+
 # 64 output channels take a kernel of their own: row counts that end inside its 32-token tiles, K of fewer k steps than
 # its 4 waves, of whole and of cut rounds of its 3 stages, strides, batch items and each output type
 @pytest.mark.parametrize("Mr,K", [(1, 64), (31, 192), (33, 832), (64, 768), (300, 3072), (8200, 1536)])
