@@ -123,6 +123,8 @@ constexpr int EK_F16 = 64;
 // k step's loads issued NSTG - 1 steps ahead of its use; the two-workgroup form stages them through registers three
 // substeps ahead, a latency a workgroup alone on its CU cannot hide.
 constexpr int EK_DEEP = 128;
+// Flag on EK_HEADS: 128-dim heads on 128 x 128 tiles, whose 4 waves take 32 tokens x all 128 channels (one head) each.
+constexpr int EK_H128 = 256;
 // s_waitcnt immediate (gfx9 layout): vmcnt vm (0-63: bits 3:0 and 15:14), expcnt not waited for, lgkmcnt lgkm (0-15)
 constexpr int waitcnt_bits(int vm, int lgkm) { return (vm & 15) | ((vm >> 4) << 14) | (7 << 4) | ((lgkm & 15) << 8); }
 typedef _Float16 f16x8v __attribute__((ext_vector_type(8)));
@@ -760,8 +762,9 @@ __device__ __forceinline__ void gemm_tile(const GemmP& p, uint32_t z, uint32_t t
     constexpr int NSTG = kDeep ? (BM == 128 ? 4 : 3) : 2; // LDS stages of the operand tiles
     constexpr int EKE = EK & 7;                 // the epilogue kind
     constexpr int NT = 64 * NW;                 // threads
-    // waves: 2 along channels x NW/2 along tokens; the 96-channel tiles 1 x NW (a wave holds whole rows)
-    constexpr int WCH = BN == 96 ? 1 : 2;
+    // waves: 2 along channels x NW/2 along tokens; the 96-channel tiles and 128-dim heads on 128-channel tiles 1 x NW
+    // (a wave holds whole rows, or a whole head)
+    constexpr int WCH = BN == 96 || (EK & EK_H128) ? 1 : 2;
     constexpr int WM = BM / (NW / WCH);         // tokens per wave
     constexpr int WC = BN / WCH;                // channels per wave
     // 8-wave tiles run v_mfma_f32_16x16x32_bf16 (16 x 16 output blocks, 32-deep substeps: 3-4% faster than the
@@ -1426,10 +1429,10 @@ __device__ __forceinline__ void gemm_tile(const GemmP& p, uint32_t z, uint32_t t
 }
 
 
-template <int BM, int BN, int NW, bool DEEP = false>
+template <int BM, int BN, int NW, int EK = 0>
 constexpr int gemm_smem()
 {
-    constexpr int LDW = BN / 2 + 4, NSTG = DEEP ? (BM == 128 ? 4 : 3) : 2;
+    constexpr int LDW = (EK & EK_H128 ? BN : BN / 2) + 4, NSTG = EK & EK_DEEP ? (BM == 128 ? 4 : 3) : 2;
     return NSTG * (BN + BM) * 64 * 2 > NW * 32 * LDW * 4 ? NSTG * (BN + BM) * 64 * 2 : NW * 32 * LDW * 4;
 }
 
@@ -1445,7 +1448,7 @@ template <int BM, int BN, bool kF8, int EK, int NW>
 __global__ __launch_bounds__(64 * NW, BM == 128 && !(EK & EK_DEEP) ? 2 : 1) __attribute__((
     amdgpu_waves_per_eu(gemm_waves_per_eu<BM, NW, EK>(), gemm_waves_per_eu<BM, NW, EK>()))) void gemm_kernel(GemmG G)
 {
-    __shared__ __attribute__((aligned(16))) uint16_t smem[gemm_smem<BM, BN, NW, (EK & EK_DEEP) != 0>() / 2];
+    __shared__ __attribute__((aligned(16))) uint16_t smem[gemm_smem<BM, BN, NW, EK>() / 2];
     uint32_t z, tm, tn;
     const GemmP& p = locate(G, xcd_order(blockIdx.x, gridDim.x), z, tm, tn);
     gemm_tile<BM, BN, kF8, EK, NW>(p, z, tm, tn, 0, int(p.K) / BK, smem, nullptr, -1);
@@ -1460,7 +1463,7 @@ __global__ __launch_bounds__(64 * NW, BM == 128 && !(EK & EK_DEEP) ? 2 : 1) __at
                                                                                             uint32_t tiles,
                                                                                             uint64_t slab)
 {
-    __shared__ __attribute__((aligned(16))) uint16_t smem[gemm_smem<BM, BN, NW, (EK & EK_DEEP) != 0>() / 2];
+    __shared__ __attribute__((aligned(16))) uint16_t smem[gemm_smem<BM, BN, NW, EK>() / 2];
     // split-major: an XCD's run of workgroups shares its splits' columns of A
     const uint32_t i = xcd_order(blockIdx.x, gridDim.x), s = i / tiles;
     uint32_t z, tm, tn;
@@ -2204,8 +2207,14 @@ GemmPlan gemm_plan(const mk_gemm_args* a, uint32_t n, uint32_t cus, bool conv)
         return best;
     }
     consider(256, 256, 1.0);
-    if (heads)
+    if (heads) {
+        // 128-dim heads on 128 x 128 tiles: 0.74 (measured, K = 3072, us on 256 x 256 tiles -> on these: 1 x (256 + 64)
+        // rows 84 -> 42, fp8 75 -> 38, 2 x (576 + 77) 162 -> 114, 1 x (1600 + 200) 164 -> 148; 1 x (1024 + 131) 97 and
+        // 100, 2 x (2304 + 64) 256 and 308, 1 x (4096 + 256) 279 and 303)
+        if (a[0].w_dtype != MK_F16)
+            consider(128, 128, 0.74);
         return best;
+    }
     consider(256, 128, 0.66);
     if (conv)
         consider(256, 192, 0.78);
@@ -2284,8 +2293,10 @@ extern "C" mk_status mk_gemm_grouped(const mk_gemm_args* a, uint32_t count, void
     const int bn = plan.bn;
     if (bn == 64 && (ek == EK_ACT || ek == EK_GLU))
         return fail(MK_ERR_UNSUPPORTED, "gemm: activation and GLU epilogues need N a multiple of 128");
-    // the heads epilogue writes one head per wave slice: 128-dim heads on 256-channel tiles, 64-dim on 128-channel
-    if (ek == EK_HEADS && !((bn == 256 && p[0].hp.hd == 128) || (bn == 128 && p[0].hp.hd == 64)))
+    // the heads epilogue writes one head per wave slice: 128-dim heads on 256-channel tiles or, a wave across the tile,
+    // on 128 x 128 ones; 64-dim heads on 128-channel tiles
+    const bool h128 = ek == EK_HEADS && p[0].hp.hd == 128 && plan.bm == 128 && bn == 128;
+    if (ek == EK_HEADS && !h128 && !((bn == 256 && p[0].hp.hd == 128) || (bn == 128 && p[0].hp.hd == 64)))
         return fail(MK_ERR_UNSUPPORTED, "gemm: heads epilogue tile width does not match the head dim");
     hipStream_t s = static_cast<hipStream_t>(stream);
     // 64 channels stored: gemm_n64_kernel up to as many rounds of its workgroups as it wins (K = 3072: 32768 rows, 4
@@ -2337,6 +2348,12 @@ extern "C" mk_status mk_gemm_grouped(const mk_gemm_args* a, uint32_t count, void
         if (ek == EK_HEADS)
             return f16(std::integral_constant<int, EK_HEADS>{});
         return f16(std::integral_constant<int, EK_GLU>{});
+    }
+    if (h128) {
+        if (f8)
+            return launch<128, 128, true, EK_HEADS | EK_H128, 4>(p, n, plan, s);
+        return deep ? launch<128, 128, false, EK_HEADS | EK_H128 | EK_DEEP, 4>(p, n, plan, s)
+                    : launch<128, 128, false, EK_HEADS | EK_H128, 4>(p, n, plan, s);
     }
     // 256-wide tiles: 8 waves (two a SIMD, 64 x 128 wave tiles), so one wave's waits (barrier, loads) leave the
     // other's MFMAs running

@@ -414,6 +414,34 @@ def test_gemm_heads_vt_behind_any_prompt(gpu, rng, row0, Mr, odt):
     assert not np.delete(got, cols, 2).any()  # the keys before and behind stay zero
 
 
+# 128-dim heads of few rows take 128 x 128 tiles, many rows 256 x 256 ones: the same rows have the same bits either way,
+# for every RoPE mode, both weight types, batch items and row counts that end inside a tile
+@pytest.mark.parametrize("mode,wdt,odt", [(0, M.BF16, M.F16), (1, M.BF16, M.BF16), (2, M.BF16, M.BF16),
+                                          (2, M.FP8, M.F16)])
+@pytest.mark.parametrize("Mr", [1, 130, 640])
+def test_gemm_heads_small_tiles_same_bits(gpu, rng, mode, wdt, odt, Mr):
+    H, K_, row0, big = 2, 192, 19, 16384
+    D, pad = H * 128, 16640
+    A = bdev(rng.standard_normal((big, K_)).astype(np.float32))
+    if wdt == M.FP8:
+        W, sc = dev(rng.integers(0, 126, (3 * D, K_)).astype(np.uint8)), dev(np.full(3 * D, 1e-3, np.float32))
+    else:
+        W, sc = bdev(rng.standard_normal((3 * D, K_)).astype(np.float32) * 0.05), None
+    b, nq = dev(rng.standard_normal(3 * D).astype(np.float32)), dev(1 + 0.1 * rng.standard_normal(128).astype(np.float32))
+    cs = dev(rng.standard_normal((pad, 128)).astype(np.float32))
+    outs = []
+    for rows in (Mr, big):
+        Q, Kd, Vt = (dev(np.zeros(H * pad * 128, np.uint16)) for _ in range(3))
+        ha = M.HeadsArgs(Q.p, Kd.p, Vt.p, H, 128, pad, pad, row0, 0, nq.p, nq.p, cs.p if mode else None, mode, 1e-6,
+                         0.3, odt)
+        gemm(A, W, bias=b, wscale=sc, epi=M.EPI_HEADS, c_dtype=M.BF16, M_=(rows, 3 * D, K_), lda=K_, w_dtype=wdt,
+             heads=ha)
+        outs.append((fetch(Q, (H, pad, 128), np.uint16)[:, :Mr], fetch(Kd, (H, pad, 128), np.uint16)[:, row0:row0 + Mr],
+                     fetch(Vt, (H, 128, pad), np.uint16)[:, :, M.vt_col(np.arange(row0, row0 + Mr))]))
+    for small, large in zip(*outs):
+        assert small.any() and np.array_equal(small, large)
+
+
 # 64-dim heads (the SDXL form: half, no norm, no RoPE) on 128-channel tiles: q | k | v and Q alone, batch 2, row
 # counts that end inside a tile and inside a 16-key group; each value within one rounding (half or bf16) of the
 # oracle's GEMM, padding rows untouched (zero)
