@@ -2155,8 +2155,8 @@ mk_status gemm_take_error(const void* stream, bool all)
 // 128 x 128 tiles is 2 per CU and an odd last tile costs half a pair; ties keep the larger tile. Convolutions also
 // have 256 x 192 tiles (8 waves, 0.78), for their 192- and 384-channel layers, and 128 x 96 tiles (4 waves on
 // 16 x 16 x 32, two workgroups a CU) for output channels that are an odd multiple of 96. The heads epilogue
-// takes 256 x 256 tiles for 128-dim heads and 128-channel tiles for 64-dim heads; fp8 weights 256-token tiles, and so
-// do half-weight convolutions.
+// takes 256 x 256 or 128 x 128 tiles for 128-dim heads and 128-channel tiles for 64-dim heads; half-weight convolutions
+// 256-token tiles.
 // 256 x 256 tiles use stream-K when whole waves leave at least 5% of the last wave's workgroups idle and
 // a tile is long (K of 6144 or more; measured, the partials' exchange costs about 24 k steps of a tile, more than the
 // balance saves on shorter tiles): the whole waves go round robin, the rest is split by k steps (at least 4 a
@@ -2169,8 +2169,8 @@ GemmPlan gemm_plan(const mk_gemm_args* a, uint32_t n, uint32_t cus, bool conv)
     const bool narrow_ok = a[0].epilogue != MK_EPI_GELU_TANH && a[0].epilogue != MK_EPI_SILU &&
                            a[0].epilogue != MK_EPI_SWIGLU && a[0].epilogue != MK_EPI_GEGLU &&
                            a[0].epilogue != MK_EPI_PAIR_SUM; // 64-wide tiles
-    // 128-token tiles: bf16 or half weights (convolutions: bf16 only, as their plans were measured)
-    const bool short_ok = !heads && (conv ? a[0].w_dtype == MK_BF16 : a[0].w_dtype != MK_FP8_E4M3);
+    // 128-token tiles (convolutions: bf16 only, as their plans were measured)
+    const bool f8 = a[0].w_dtype == MK_FP8_E4M3, short_ok = !heads && (!conv || a[0].w_dtype == MK_BF16);
     auto tiles_of = [&](int bm, int bn) {
         uint64_t t = 0;
         for (uint32_t i = 0; i < n; ++i)
@@ -2223,7 +2223,9 @@ GemmPlan gemm_plan(const mk_gemm_args* a, uint32_t n, uint32_t cus, bool conv)
     if (narrow_ok)
         consider(256, 64, 0.62);
     if (short_ok)
-        consider(128, 128, 0.67);
+        // fp8 weights: 0.76 (their conversion; us on the best 256-token tiles -> on these: 600 x 12288 x 3072 74 -> 58, 2048
+        // x 10240 x 1280 GEGLU 76 -> 62, 1024 x 3072 x 3072 38 -> 35; 1024 x 12288 x 3072 76 and 89)
+        consider(128, 128, f8 ? 0.76 : 0.67);
     if (best.cost < 0) // N not a multiple of 128 with an activation or GLU: the dispatch rejects it
         consider(256, 64, 0.62);
     // Few rows and long K: split each 128 x 128 tile's k steps over S workgroups (gemm_split_kernel), at most one a CU.
@@ -2318,6 +2320,9 @@ extern "C" mk_status mk_gemm_grouped(const mk_gemm_args* a, uint32_t count, void
     const bool deep = !f8 && plan.tiles <= uint64_t(cus > 0 ? cus : 1);
     auto narrow = [&](auto e_c) -> mk_status {
         constexpr int E = decltype(e_c)::value;
+        if constexpr (!(E & EK_F16))
+            if (f8) // 128 x 128 (256 x 128 below)
+                return launch<128, 128, true, E, 4>(p, n, plan, s);
         if (plan.bm == 128)
             return deep ? launch<128, 128, false, E | EK_DEEP, 4>(p, n, plan, s)
                         : launch<128, 128, false, E, 4>(p, n, plan, s);

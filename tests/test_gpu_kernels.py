@@ -442,6 +442,30 @@ def test_gemm_heads_small_tiles_same_bits(gpu, rng, mode, wdt, odt, Mr):
         assert small.any() and np.array_equal(small, large)
 
 
+# fp8 weights on 128 x 128 tiles (launches between the split ones and whole rounds of 256 x 256): the last row tile cut,
+# each epilogue, against the product of the decoded weights
+@pytest.mark.parametrize("epi", [M.EPI_STORE, M.EPI_GATE_ADD, M.EPI_GELU_TANH, M.EPI_SWIGLU])
+def test_gemm_fp8_short_tiles(gpu, rng, epi):
+    Mr, N, K = 600, 1280, 192
+    A = R.bf16_round(rng.standard_normal((Mr, K)).astype(np.float32))
+    codes = rng.integers(0, 126, (N, K)).astype(np.uint8) | (rng.integers(0, 2, (N, K)) << 7).astype(np.uint8)
+    scale = rng.uniform(0.5, 1.5, N).astype(np.float32) * 1e-3
+    b, gate = rng.standard_normal(N).astype(np.float32) * 0.3, rng.standard_normal(N).astype(np.float32)
+    glu, resid = epi == M.EPI_SWIGLU, epi == M.EPI_GATE_ADD
+    F, out16 = N // 2 if glu else N, epi in (M.EPI_GELU_TANH, M.EPI_SWIGLU)
+    X = rng.standard_normal((Mr, F)).astype(np.float32)
+    out = dev(X if resid else np.zeros((Mr, F), np.uint16 if out16 else np.float32))
+    gemm(bdev(A), dev(codes), bias=dev(b), wscale=dev(scale), c=out, c_dtype=M.BF16 if out16 else M.F32, epi=epi,
+         M_=(Mr, N, K), lda=K, ldc=F, w_dtype=M.FP8, gate=dev(gate) if resid else None)
+    got = fetch_bf16(out, (Mr, F)) if out16 else fetch(out, (Mr, F))
+    y = A.astype(np.float64) @ (R.e4m3_table()[codes] * scale[:, None]).T.astype(np.float64) + b
+    want = {M.EPI_STORE: lambda: y, M.EPI_GATE_ADD: lambda: X + gate * y,
+            M.EPI_GELU_TANH: lambda: R.gelu_tanh(y.astype(np.float32)),
+            M.EPI_SWIGLU: lambda: y[:, :F] / (1 + np.exp(-y[:, :F])) * y[:, F:]}[epi]()
+    tol = 1e-5 + (2 ** -8 if out16 else 0)  # fp32 sums, one rounding of 16-bit outputs
+    assert np.abs(got - want).max() <= tol * max(np.abs(want).max(), np.abs(y).max())
+
+
 # 64-dim heads (the SDXL form: half, no norm, no RoPE) on 128-channel tiles: q | k | v and Q alone, batch 2, row
 # counts that end inside a tile and inside a 16-key group; each value within one rounding (half or bf16) of the
 # oracle's GEMM, padding rows untouched (zero)
