@@ -2229,21 +2229,22 @@ GemmPlan gemm_plan(const mk_gemm_args* a, uint32_t n, uint32_t cus, bool conv)
     if (best.cost < 0) // N not a multiple of 128 with an activation or GLU: the dispatch rejects it
         consider(256, 64, 0.62);
     // Few rows and long K: split each 128 x 128 tile's k steps over S workgroups (gemm_split_kernel), at most one a CU.
-    // In us, a k step takes 0.42, a split adds 0.3 and its slab's write and read at 2.5 TB/s, the reduce launch 3; S is
+    // In us, a k step takes 0.42 (fp8 weights 0.6), a split adds 0.3 and its slab at 1.8 TB/s, the reduce launch 3; S is
     // the one with the least sum, 1 included. Measured (isolated launches, whole tiles -> the rule's S; the best S of a
-    // sweep over 2-16 is within 10%): 77 x 3072 x 12288 98 -> 25 us (S 10), 320 x 3072 x 12288 101 -> 48 (3), fp8 128 x
-    // 3072 x 12288 120 -> 24 (10), 64 x 3072 x 3584 19.9 -> 12.5 (6), 77 x 12288 x 3072 33 -> 28 (2), f16 512 x 1280 x
-    // 5120 34 -> 20 (5); 512 x 1280 x 1280 stays whole (13.6 against 14.0). More than 512 rows stay whole too, so that
+    // sweep over 2-16 is within 10%): 77 x 3072 x 12288 98 -> 24 us (S 10), 320 x 3072 x 12288 100 -> 47 (3), fp8 128 x
+    // 3072 x 12288 120 -> 24 (10), 64 x 3072 x 3584 19.7 -> 12.7 (6), 77 x 12288 x 3072 33 -> 27 (2), f16 512 x 1280 x
+    // 5120 34 -> 19 (4), 600 x 3072 x 12288 110 -> 72 (2), 960 x 1280 x 5120 35 -> 23 (3); 512 x 1280 x 1280 stays whole
+    // (13.6 against 14.0 in two), so does 640 x 3072 x 3584 (23.6 against 27.0). 1024 rows and more stay whole, so that
     // the parts of an image's rows launched apart get the bits of one launch.
     uint64_t rows = 0;
     for (uint32_t i = 0; i < n; ++i)
         rows += uint64_t(a[i].M) * a[i].batch;
-    if (!conv && N % 128 == 0 && rows <= 512) {
+    if (!conv && N % 128 == 0 && rows < 1024) {
         const uint64_t cap = cus / std::max<uint64_t>(1, tiles_of(128, 128));
-        const double slab = double(rows) * N * 4, whole = 0.42 * double(kt);
+        const double slab = double(rows) * N * 4, whole = (f8 ? 0.6 : 0.42) * double(kt);
         double least = whole;
         for (uint64_t sp = 2; sp <= cap && sp <= kt && double(sp) * slab <= double(gemm_detail::kSplitBytes); ++sp) {
-            const double t = whole / double(sp) + 3.0 + double(sp) * (0.3 + slab / 2.5e6);
+            const double t = whole / double(sp) + 3.0 + double(sp) * (0.3 + slab / 1.8e6);
             if (t < least) {
                 least = t;
                 best.splits = int(sp);
