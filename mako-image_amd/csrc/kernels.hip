@@ -3,6 +3,8 @@
 // patchify, and the counter-RNG fill. Each is a wave64 kernel with 16-byte coalesced accesses where the row allows.
 #include "common.hpp"
 
+#include <type_traits>
+
 #include <cmath>
 #include <algorithm>
 #include <mutex>
@@ -502,30 +504,33 @@ __global__ __launch_bounds__(256) void gemv_kernel(const float* __restrict__ x, 
     }
 }
 
-// GEMV for one row with K = 512 * KI: each wave computes 4 outputs with all 4 * KI of its 16-byte weight loads
-// issued first; while they are in flight the workgroup (8 waves, 32 outputs) converts x' to bf16 in LDS once (each
-// wave converting the whole row itself cost more VALU time than the dot products), and the dot products take the
-// bf16 pairs as they are (v_dot2_f32_bf16).
-template <int KI>
-__global__ __launch_bounds__(512) void gemv1_kernel(const float* __restrict__ x, const uint16_t* __restrict__ w,
-                                                    const float* __restrict__ bias, uint32_t N, float* __restrict__ y,
-                                                    int silu_x)
+// GEMV for R rows (1 or 2) with K = 512 * KI: each wave computes 2 outputs with all 2 * KI of its 16-byte weight loads issued
+// first; while they are in flight the workgroup (8 waves, 16 outputs) converts x' to bf16 in LDS once (each wave
+// converting the whole row itself cost more VALU time than the dot products), and the dot products take the bf16 pairs
+// as they are (v_dot2_f32_bf16). HBM-bound once the launch fills the chip, which 16 outputs a workgroup do from 4096
+// outputs on; 4 outputs a wave measured slower at every size (1 x 3072 x 3072 7.5 against 5.8 us, 1 x 368640 x 3072 324
+// against 312 us, 7.2 TB/s), one the same. Two rows on this form instead of gemv_kernel (scalar fp32 products, its loads
+// behind the row's staging): 4096 x 4096 42 -> 9.4 us, 16384 x 4096 70 -> 31 us.
+template <int KI, int R>
+__global__ __launch_bounds__(512) void gemv_rows_kernel(const float* __restrict__ x, const uint16_t* __restrict__ w,
+                                                        const float* __restrict__ bias, uint32_t N,
+                                                        float* __restrict__ y, int silu_x)
 {
-    constexpr uint32_t K = 512 * KI;
-    __shared__ __attribute__((aligned(16))) uint16_t xs[K];
-    const uint32_t lane = threadIdx.x & 63, n0 = (blockIdx.x * 8 + (threadIdx.x >> 6)) * 4;
-    // the wave's 4 weight rows first (16-byte chunks, all in flight; rows past N read the last row), as nontemporal
+    constexpr uint32_t K = 512 * KI, J = 2;
+    __shared__ __attribute__((aligned(16))) uint16_t xs[R * K];
+    const uint32_t lane = threadIdx.x & 63, n0 = (blockIdx.x * 8 + (threadIdx.x >> 6)) * J;
+    // the wave's J weight rows first (16-byte chunks, all in flight; rows past N read the last row), as nontemporal
     // loads: the stacked modulation matrix streams through once a step and is not kept in the caches
-    u32x4 wv[4][KI];
+    u32x4 wv[J][KI];
     if (n0 < N)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (uint32_t j = 0; j < J; ++j)
 #pragma unroll
             for (int i = 0; i < KI; ++i)
                 wv[j][i] = __builtin_nontemporal_load(
                     reinterpret_cast<const u32x4*>(w + uint64_t(min(n0 + j, N - 1)) * K + lane * 8 + 512 * i));
-    // meanwhile the input row, once a workgroup, as the GEMMs' bf16 activation operand (silu first when asked)
-    for (uint32_t k = threadIdx.x; k < K / 2; k += 512) {
+    // meanwhile the input rows, once a workgroup, as the GEMMs' bf16 activation operand (silu first when asked)
+    for (uint32_t k = threadIdx.x; k < R * K / 2; k += 512) {
         float a = x[2 * k], b = x[2 * k + 1];
         if (silu_x) {
             a = a / (1.0f + __expf(-a));
@@ -538,27 +543,29 @@ __global__ __launch_bounds__(512) void gemv1_kernel(const float* __restrict__ x,
         return;
     // bf16 pairs straight into v_dot2_f32_bf16 (exact products, fp32 sums)
     typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2;
-    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    float acc[R][J] = {};
 #pragma unroll
-    for (int i = 0; i < KI; ++i) {
-        const u32x4 xv = *reinterpret_cast<const u32x4*>(&xs[lane * 8 + 512 * i]);
+    for (int i = 0; i < KI; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int r = 0; r < R; ++r) {
+            const u32x4 xv = *reinterpret_cast<const u32x4*>(&xs[r * K + lane * 8 + 512 * i]);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const uint32_t wu = wv[j][i][e], xu = xv[e];
-                acc[j] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, wu),
-                                                         __builtin_bit_cast(bf16x2, xu), acc[j], false);
-            }
-    }
+            for (uint32_t j = 0; j < J; ++j)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-        acc[j] = wave_sum(acc[j]);
-    if (lane < 4) {
-        const float v = lane == 0 ? acc[0] : lane == 1 ? acc[1] : lane == 2 ? acc[2] : acc[3];
-        if (n0 + lane < N)
-            y[n0 + lane] = v + (bias ? bias[n0 + lane] : 0.0f);
-    }
+                for (int e = 0; e < 4; ++e) {
+                    const uint32_t wu = wv[j][i][e], xu = xv[e];
+                    acc[r][j] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, wu),
+                                                                __builtin_bit_cast(bf16x2, xu), acc[r][j], false);
+                }
+        }
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (uint32_t j = 0; j < J; ++j) {
+            const float v = wave_sum(acc[r][j]);
+            if (lane == j && n0 + j < N)
+                y[uint64_t(r) * N + n0 + j] = v + (bias ? bias[n0 + j] : 0.0f);
+        }
 }
 
 template <int kOp>
@@ -1139,13 +1146,20 @@ mk_status mk_gemv(const float* x, uint32_t rows, uint32_t K, const void* w, cons
     if (!x || !w || !y || rows == 0 || rows > 4 || K % 8 || uint64_t(rows) * K * 4 > 64 * 1024)
         return fail(MK_ERR_ARG, "gemv: null pointer, rows not 1..4, K not a multiple of 8 or rows*K over 16384");
     const uint16_t* wb = static_cast<const uint16_t*>(w);
-    const dim3 grid(cdiv(N, 16)), grid1(cdiv(N, 32));
-    if (rows == 1 && K == 3072)
-        gemv1_kernel<6><<<grid1, 512, 0, S(stream)>>>(x, wb, bias, N, y, silu_x);
-    else if (rows == 1 && K == 4096)
-        gemv1_kernel<8><<<grid1, 512, 0, S(stream)>>>(x, wb, bias, N, y, silu_x);
-    else if (rows == 1 && K == 2048)
-        gemv1_kernel<4><<<grid1, 512, 0, S(stream)>>>(x, wb, bias, N, y, silu_x);
+    const dim3 grid(cdiv(N, 16));
+    auto rows_of = [&](auto ki_c) {
+        constexpr int KI = decltype(ki_c)::value;
+        if (rows == 1)
+            gemv_rows_kernel<KI, 1><<<grid, 512, 0, S(stream)>>>(x, wb, bias, N, y, silu_x);
+        else
+            gemv_rows_kernel<KI, 2><<<grid, 512, 0, S(stream)>>>(x, wb, bias, N, y, silu_x);
+    };
+    if (rows <= 2 && K == 3072)
+        rows_of(std::integral_constant<int, 6>{});
+    else if (rows <= 2 && K == 4096)
+        rows_of(std::integral_constant<int, 8>{});
+    else if (rows <= 2 && K == 2048)
+        rows_of(std::integral_constant<int, 4>{});
     else
         gemv_kernel<<<grid, 256, rows * K * 4, S(stream)>>>(x, rows, K, wb, bias, N, y, silu_x);
     MK_LAUNCH_CHECK("gemv");

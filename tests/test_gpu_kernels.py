@@ -1041,6 +1041,22 @@ def test_gemv_modulation(gpu, rng, rows, K, silu):
     assert maxrel(fetch(y, (rows, N)), want) < 1e-5
 
 
+# two rows share the one-row kernel's form for K in {2048, 3072, 4096}, three take the LDS-staged one: one output, a
+# workgroup's last pair cut
+@pytest.mark.parametrize("rows,K", [(2, 2048), (2, 4096), (3, 3072)])
+@pytest.mark.parametrize("N", [1, 17])
+def test_gemv_few_outputs(gpu, rng, rows, K, N):
+    x = rng.standard_normal((rows, K)).astype(np.float32)
+    W = R.bf16_round(rng.standard_normal((N, K)).astype(np.float32) * 0.02)
+    y = dev(np.full(rows * N + 4, 7.5, np.float32))
+    M.call("mk_gemv", dev(x).p, rows, K, bdev(W).p, None, N, y.p, 1, None)
+    M.sync()
+    got = fetch(y, (rows * N + 4,))
+    want = R.gemm(R.silu(x), W, None)
+    assert np.abs(got[:rows * N].reshape(rows, N) - want).max() < 1e-5 * max(1.0, np.abs(want).max())  # fp32 sums
+    assert (got[rows * N:] == 7.5).all()
+
+
 @pytest.mark.parametrize("n", [12, 260, 640, 1280, 3072, 4096])  # 1, 2, 3, 5, 12 and 16 float4s a lane
 def test_norms(gpu, rng, n):
     rows = 70
