@@ -31,7 +31,8 @@ struct AttnP {
     uint16_t* out;
     uint32_t heads, group, batch, n_q, q_pad, n_k, k_pad, q_pos0, block; // group: query heads a key / value head
     int64_t ldo, so;
-    float c; // scale * log2(e)
+    float c;      // |scale| * log2(e)
+    uint32_t neg; // the scale is negative
     // keys [hole[b][0], hole[b][1]) of batch item b are masked (a shorter prompt's padding rows); empty: none
     uint32_t hole[kMaxHoleBatch][2];
     uint32_t out_f16; // the output as IEEE half (the input of a GEMM over half weights), else bf16
@@ -39,9 +40,9 @@ struct AttnP {
 
 constexpr int kKT = 64; // keys per tile
 // Lazy rescaling: the running max m the exponentials use moves only when a score exceeds it by more than kLazy (log2
-// units; the unit-scale path notices it as a row-sum part above 2^kLazy), so P stays near or below 256 (exact enough
+// units; noticed as a row-sum part above 2^kLazy), so P stays near or below 256 (exact enough
 // in bf16, far from fp32 overflow) and the output is rescaled on few tiles.
-constexpr float kLazy = 8.0f, kLazyP = 256.0f; // kLazyP = 2^kLazy
+constexpr float kLazyP = 256.0f; // 2^kLazy, kLazy = 8
 
 typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2;
 
@@ -88,11 +89,14 @@ template <> struct Elem<true> {
     }
 };
 
-// U: K carries the softmax scale in log2 units (scale 0 at the API). The running max then enters the S^T MFMAs as
-// one more 16-deep product, a constant fragment of ones (K side, dim 0) times a fragment holding -m (Q side), so
-// S - m comes out of the matrix core: the softmax needs no per-score multiply-add, and the row sums are taken on the
-// bf16 probabilities the P V product uses (v_dot2 against ones), which halves those adds too. m is kept
-// bf16-representable so the product subtracts it exactly.
+// The running max enters the S^T MFMAs as one more 16-deep product, a constant fragment of ones (K side, dim 0) times a
+// fragment holding -m (Q side), so S - m comes out of the matrix core, and the row sums are taken on the 16-bit
+// probabilities the P V product uses (v_dot2 against ones), which halves those adds too. m is kept representable in the
+// type so the product subtracts it exactly.
+// U: K carries the softmax scale in log2 units (scale 0 at the API), so the softmax needs no per-score multiply at all;
+// a general scale multiplies each S - m by c. (The general scale had a tile of its own, a max, a multiply-add and an
+// add a score between the MFMAs instead of in their shadow: 493 -> 463 us for 2 x 24 heads of 128 over 4352 rows, 1006
+// TFLOP/s.)
 // NW waves a workgroup (32 queries each): 4, or 2 for launches of few query blocks (64-dim heads), whose 64-query
 // workgroups then spread over every CU, four a CU.
 template <int D, bool U, bool F16, bool HOLE, int NW = 4>
@@ -100,7 +104,6 @@ __global__ __launch_bounds__(64 * NW, 2) __attribute__((amdgpu_waves_per_eu(2, 2
 {
     typedef Elem<F16> X;
     typedef typename X::v8 V8;
-    typedef typename X::e E;
     constexpr int DS = D / 16, DT = D / 32, KC = D / 8, QB = 32 * NW; // QB: queries a workgroup
     constexpr int RK = kKT * KC / (64 * NW), RV = D * 8 / (64 * NW);
     static_assert(NW == 4 || NW == 2, "4 or 2 waves a workgroup");
@@ -130,12 +133,6 @@ __global__ __launch_bounds__(64 * NW, 2) __attribute__((amdgpu_waves_per_eu(2, 2
         hole_lo = bi < uint32_t(kMaxHoleBatch) ? int(p.hole[bi][0]) : 0;
         hole_hi = bi < uint32_t(kMaxHoleBatch) ? int(p.hole[bi][1]) : 0;
     }
-    auto in_hole = [&](int key) { return HOLE && key >= hole_lo && key < hole_hi; };
-    // keys [k0, k0 + n) reach into the hole (the general path masks them score by score; the scale-0 path through
-    // the matrix core, below)
-    auto hits_hole = [&](int k0, int n) {
-        return HOLE && !U && hole_lo < hole_hi && k0 < hole_hi && k0 + n > hole_lo;
-    };
     const int64_t bh = int64_t(bi) * p.heads + head, bkv = int64_t(bi) * (p.heads / p.group) + head / p.group;
     const uint16_t* Q = p.q + bh * p.q_pad * D;
     const uint16_t* K = p.k + bkv * p.k_pad * D;
@@ -148,6 +145,10 @@ __global__ __launch_bounds__(64 * NW, 2) __attribute__((amdgpu_waves_per_eu(2, 2
 #pragma unroll
         for (int ds = 0; ds < DS; ++ds)
             qf[ds] = *reinterpret_cast<const V8*>(Q + int64_t(qi) * D + ds * 16 + hk * 8);
+        if (!U && p.neg) // a negative scale: -q with the scale's magnitude
+#pragma unroll
+            for (int ds = 0; ds < DS; ++ds)
+                qf[ds] = __builtin_bit_cast(V8, __builtin_bit_cast(u32x4, qf[ds]) ^ 0x80008000u);
     }
     // K / V^T tiles go to LDS by buffer loads (resources over the head's rows; lane byte offsets select key / dim and
     // chunk, the tile's key offset is a scalar): unlike the global form they leave the LDS counter alone.
@@ -182,127 +183,49 @@ __global__ __launch_bounds__(64 * NW, 2) __attribute__((amdgpu_waves_per_eu(2, 2
             buf_load_lds16(rsV, (lds_void*)&sV(buf)[(i * NW + wave_s) * 512], ov[i], k0 * 2);
     };
     // S^T of a 32-key half of a tile: value r <-> key 8(r/4) + 4hk + r%4 of the half
-    V8 kone = {}, qm = {}; // U: ones at dim 0 (K side); -m at dim 0 (Q side), lanes of the first k half
+    // ones at dim 0 (K side); -m at dim 0 (Q side), lanes of the first k half. A general scale's scores are unscaled
+    // products, which can pass the half range: m is then the sum of two bf16 values (dims 0 and 2; 16 bits, so that a
+    // score of 10^5 in log2 units is still met to half a unit), and this one product bf16
+    typedef Elem<F16 && U> XM;
+    typedef typename XM::v8 MV8;
+    typedef typename XM::e ME;
+    MV8 kone = {}, qm = {};
     if (hk == 0)
-        kone[0] = (E)1.0f;
-    // U with a masked key range: the same product also adds bias(key) x 1 at dim 1, bias -inf for the masked keys
+        kone[0] = kone[2] = (ME)1.0f;
+    // a masked key range: the same product also adds bias(key) x 1 at dim 1, bias -inf for the masked keys
     // (0 otherwise), so their scores leave the matrix core as -inf (lanes of the first k half hold dims 0 .. 7)
-    if (HOLE && U && hk == 0)
-        qm[1] = (E)1.0f;
+    if (HOLE && hk == 0)
+        qm[1] = (ME)1.0f;
     auto kbias = [&](int key) {
-        V8 kb = kone;
+        MV8 kb = kone;
         if (hk == 0 && key >= hole_lo && key < hole_hi)
-            kb[1] = (E)(-__builtin_inff());
+            kb[1] = (ME)(-__builtin_inff());
         return kb;
     };
     f32x16 oacc[DT];
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
         oacc[dt] = f32x16{};
-    float m = U ? 0.0f : -1e30f, l = 0.0f;
+    float m = 0.0f, l = 0.0f;
+    // 2^(c x): the unit scale's scores are in log2 units already
+    const float c = p.c;
+    auto exp_c = [&](float x) { return __builtin_amdgcn_exp2f(U ? x : x * c); };
     const int qpos = int(p.q_pos0) + q0 + r32;
     const bool wave_causal = uint32_t(int(p.q_pos0) + q0) < p.block;
-    auto softmax = [&](f32x16& sacc, int k0, u32x4 (&pb)[2]) {
-        if (k0 + 32 > int(p.n_k) || (wave_causal && k0 + 31 > int(p.q_pos0) + q0) || hits_hole(k0, 32)) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int key = k0 + 8 * (r / 4) + 4 * hk + (r % 4);
-                if (key >= int(p.n_k) || (uint32_t(qpos) < p.block && key > qpos) || in_hole(key))
-                    sacc[r] = -__builtin_inff();
-            }
-        }
-        const float mx = max_xor32(max16(sacc)) * p.c;
-        if (__any(mx > m + kLazy)) {
-            const float mn = fmaxf(m, mx);
-            const float alpha = __builtin_amdgcn_exp2f(m - mn);
-            m = mn;
-            l *= alpha;
-#pragma unroll
-            for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    oacc[dt][r] *= alpha;
-        }
-        float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const float e = __builtin_amdgcn_exp2f(fmaf(sacc[r], p.c, -m));
-            sacc[r] = e;
-            sum[r % 4] += e;
-        }
-        l += (sum[0] + sum[1]) + (sum[2] + sum[3]);
-#pragma unroll
-        for (int st = 0; st < 2; ++st) {
-            const int o = 8 * st;
-            pb[st] = u32x4{X::pack(sacc[o], sacc[o + 1]), X::pack(sacc[o + 2], sacc[o + 3]),
-                           X::pack(sacc[o + 4], sacc[o + 5]), X::pack(sacc[o + 6], sacc[o + 7])};
-        }
-    };
     issue(0, 0);
     f32x16 s_a, s_b;
-    // General scale: one 64-key tile from buffer `buf` (a constant: the loop is unrolled by two, so the LDS reads and
-    // the next tile's loads provably touch different buffers and the reads wait for nothing but themselves). The
-    // tile's 32 fragment reads (K of both 32-key halves interleaved, then V of each half) stream four ahead of the
-    // MFMAs that use them, in a fixed order (fenced); the two halves' S^T products alternate so neither accumulator
-    // chain waits on its previous MFMA.
     constexpr int LA = 4; // fragment reads in flight ahead of their MFMA
-    auto tile = [&](int t, auto buf_c) {
-        constexpr int buf = decltype(buf_c)::value;
-        __builtin_amdgcn_s_waitcnt(0); // tile t resident
-        __syncthreads();               // ... for every wave, and every wave done with tile t - 1's buffer
-        issue(t + 1, buf ^ 1);         // past the end: the last tile again (discarded)
-        V8 fk[2 * DS], fv[4 * DT];
-        // read g: K fragments g < 2 DS as (ds, half) pairs, then V fragments of half 0, then half 1
-        auto rd = [&](int g) {
-            if (g < 2 * DS) {
-                const int ds = g / 2, kt = g % 2, key = kt * 32 + r32, c = kswz(key, ds * 2 + hk);
-                fk[g] = *reinterpret_cast<const V8*>(&sK(buf)[key * D + c * 8]);
-            } else if (g < 2 * DS + 4 * DT) {
-                const int j = g - 2 * DS, kt = j / (2 * DT), dt = (j % (2 * DT)) % DT, st = (j % (2 * DT)) / DT;
-                const int d = dt * 32 + r32, s2 = 2 * kt + st;
-                fv[j] = *reinterpret_cast<const V8*>(&sV(buf)[d * kKT + (((2 * s2 + hk) ^ ((d >> 1) & 7)) << 3)]);
-            }
-        };
-#pragma unroll
-        for (int g = 0; g < LA; ++g)
-            rd(g);
-        __builtin_amdgcn_sched_barrier(0);
-        s_a = f32x16{};
-        s_b = f32x16{};
-#pragma unroll
-        for (int g = 0; g < 2 * DS; ++g) {
-            f32x16& acc = g % 2 ? s_b : s_a;
-            acc = X::mfma(fk[g], qf[g / 2], acc, 0, 0, 0);
-            __builtin_amdgcn_sched_barrier(0);
-            rd(g + LA);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        u32x4 pb[2];
-        auto pv = [&](int kt) {
-#pragma unroll
-            for (int j = 0; j < 2 * DT; ++j) {
-                const int dt = j % DT, st = j / DT;
-                oacc[dt] = X::mfma(fv[kt * 2 * DT + j], __builtin_bit_cast(V8, pb[st]),
-                                                                   oacc[dt], 0, 0, 0);
-                __builtin_amdgcn_sched_barrier(0);
-                rd(2 * DS + kt * 2 * DT + j + LA);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        };
-        softmax(s_a, t * kKT, pb);
-        pv(0);
-        softmax(s_b, t * kKT + 32, pb);
-        pv(1);
-    };
-    // U: one 64-key tile with the softmax work in the matrix core's shadow. The scores arrive as S - m, so each
-    // half's probabilities are computed speculatively, before its row max is known: P = 2^(S - m) is what the tile
-    // needs whenever no score exceeds m by more than kLazy. The exponentials, conversions and row sums of half a then
+    // One 64-key tile from buffer `buf` (a constant: the loop is unrolled by two, so the LDS reads and the next tile's
+    // loads provably touch different buffers and the reads wait for nothing but themselves), the softmax work in the
+    // matrix core's shadow. The tile's 32 fragment reads stream LA ahead of the MFMAs that use them, in a fixed order
+    // (fenced). The scores arrive as S - m, so each half's probabilities are computed speculatively, before its row max
+    // is known: P = 2^(c (S - m)) is what the tile needs whenever no score exceeds m by more than kLazy in log2 units. The exponentials, conversions and row sums of half a then
     // run in chunks between the S^T MFMAs of half b, those of half b between the P V MFMAs of half a, and the lane's
     // part of the row sum only decides afterwards whether a half is redone against a new m (the first half of the
     // pass, and the rare tiles whose max jumps: a score more than kLazy above m puts that sum above 2^kLazy). EDGE
     // tiles (ragged key end, causal diagonal, a masked key range) mask scores in the chunks.
     constexpr int CH = 16 / DS;                  // scores per chunk: DS S^T MFMAs (= 2 DT P V MFMAs) per half
-    auto tile_u = [&](int t, auto buf_c, auto edge_c) {
+    auto tile = [&](int t, auto buf_c, auto edge_c) {
         constexpr int buf = decltype(buf_c)::value;
         constexpr bool EDGE = decltype(edge_c)::value;
         __builtin_amdgcn_s_waitcnt(0);
@@ -336,7 +259,7 @@ __global__ __launch_bounds__(64 * NW, 2) __attribute__((amdgpu_waves_per_eu(2, 2
                     sc[2 * j] = x0;
                     sc[2 * j + 1] = x1;
                 }
-                pw[j] = X::pack(__builtin_amdgcn_exp2f(x0), __builtin_amdgcn_exp2f(x1));
+                pw[j] = X::pack(exp_c(x0), exp_c(x1));
                 ls = X::sum2(pw[j], ls);
                 // pinned here: the redo path overwrites them, so the compiler would otherwise sink the
                 // speculative work out of the MFMA shadow into the path that keeps it
@@ -347,12 +270,13 @@ __global__ __launch_bounds__(64 * NW, 2) __attribute__((amdgpu_waves_per_eu(2, 2
         // the old m, and redoes the half's probabilities and row sum
         auto redo = [&](f32x16& sc, uint32_t (&pw)[8], float& lh, bool first, f32x16* other) {
             const float mx = max_xor32(max16(sc));
-            const float mn = float((E)(m + (first ? mx : fmaxf(mx, 0.0f))));
+            const float mt = m + (first ? mx : fmaxf(mx, 0.0f)), m1 = float((ME)mt);
+            const float m2 = U ? 0.0f : float((ME)(mt - m1)), mn = m1 + m2;
             const float dm = mn - m;
-            const float alpha = first ? 1.0f : __builtin_amdgcn_exp2f(-dm);
+            const float alpha = first ? 1.0f : exp_c(-dm);
             m = mn;
             if (hk == 0)
-                qm[0] = (E)(-m);
+                qm[0] = (ME)(-m1), qm[2] = (ME)(-m2);
             l *= alpha;
 #pragma unroll
             for (int r = 0; r < 16; ++r)
@@ -369,7 +293,7 @@ __global__ __launch_bounds__(64 * NW, 2) __attribute__((amdgpu_waves_per_eu(2, 2
             float ls = 0.0f;
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
-                pw[j] = X::pack(__builtin_amdgcn_exp2f(sc[2 * j]), __builtin_amdgcn_exp2f(sc[2 * j + 1]));
+                pw[j] = X::pack(exp_c(sc[2 * j]), exp_c(sc[2 * j + 1]));
                 ls = X::sum2(pw[j], ls);
             }
             lh = ls;
@@ -379,7 +303,7 @@ __global__ __launch_bounds__(64 * NW, 2) __attribute__((amdgpu_waves_per_eu(2, 2
         for (int g = 0; g < LA; ++g)
             rd(g);
         __builtin_amdgcn_sched_barrier(0);
-        s_a = X::mfma(HOLE ? kbias(k0 + r32) : kone, qm, f32x16{}, 0, 0, 0);
+        s_a = XM::mfma(HOLE ? kbias(k0 + r32) : kone, qm, f32x16{}, 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
         // the next tile's direct loads (past the end: the last tile again, discarded) go out one after each S^T
         // MFMA of half a, not as one burst after the barrier (a burst from every wave stalls their issue)
@@ -395,7 +319,7 @@ __global__ __launch_bounds__(64 * NW, 2) __attribute__((amdgpu_waves_per_eu(2, 2
                 dma1(t + 1, buf ^ 1, i);
             __builtin_amdgcn_sched_barrier(0);
         }
-        s_b = X::mfma(HOLE ? kbias(k0 + 32 + r32) : kone, qm, f32x16{}, 0, 0, 0);
+        s_b = XM::mfma(HOLE ? kbias(k0 + 32 + r32) : kone, qm, f32x16{}, 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
         uint32_t pa[8], pbw[8];
         float la = 0.0f, lb = 0.0f;
@@ -443,30 +367,20 @@ __global__ __launch_bounds__(64 * NW, 2) __attribute__((amdgpu_waves_per_eu(2, 2
         }
     };
     int t = 0;
-    if constexpr (U) {
-        // a tile needs masking when it passes the key end or, under the causal prefix, reaches past the wave's
-        // first query
-        auto run = [&](int tt, auto buf_c) {
-            const int e = tt * kKT + kKT - 1;
-            if (e >= int(p.n_k) || (wave_causal && e > int(p.q_pos0) + q0) || hits_hole(tt * kKT, kKT))
-                tile_u(tt, buf_c, std::true_type{});
-            else
-                tile_u(tt, buf_c, std::false_type{});
-        };
-        for (; t + 1 < ntiles; t += 2) {
-            run(t, std::integral_constant<int, 0>{});
-            run(t + 1, std::integral_constant<int, 1>{});
-        }
-        if (t < ntiles)
-            run(t, std::integral_constant<int, 0>{});
-    } else {
-        for (; t + 1 < ntiles; t += 2) {
-            tile(t, std::integral_constant<int, 0>{});
-            tile(t + 1, std::integral_constant<int, 1>{});
-        }
-        if (t < ntiles)
-            tile(t, std::integral_constant<int, 0>{});
+    // a tile needs masking when it passes the key end or, under the causal prefix, reaches past the wave's first query
+    auto run = [&](int tt, auto buf_c) {
+        const int e = tt * kKT + kKT - 1;
+        if (e >= int(p.n_k) || (wave_causal && e > int(p.q_pos0) + q0))
+            tile(tt, buf_c, std::true_type{});
+        else
+            tile(tt, buf_c, std::false_type{});
+    };
+    for (; t + 1 < ntiles; t += 2) {
+        run(t, std::integral_constant<int, 0>{});
+        run(t + 1, std::integral_constant<int, 1>{});
     }
+    if (t < ntiles)
+        run(t, std::integral_constant<int, 0>{});
     __builtin_amdgcn_s_waitcnt(0);
 
     const float lt = add_xor32(l);
@@ -523,7 +437,7 @@ mk_status attention_to(const void* q, const void* k, const void* vt, void* out, 
     AttnP p{static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(k), static_cast<const uint16_t*>(vt),
             static_cast<uint16_t*>(out), heads, heads / kv_heads, batch, n_q, q_pad, n_k, k_pad, q_pos0, block, ldo,
             stride_o,
-            scale * 1.4426950408889634f, {}, out_dtype == MK_F16 ? 1u : 0u};
+            __builtin_fabsf(scale) * 1.4426950408889634f, scale < 0.0f ? 1u : 0u, {}, out_dtype == MK_F16 ? 1u : 0u};
     if (key_hole)
         for (uint32_t b = 0; b < batch; ++b) {
             p.hole[b][0] = key_hole[2 * b];

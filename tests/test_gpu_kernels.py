@@ -1315,6 +1315,41 @@ def test_attention_masked_key_range(gpu, rng, d, Tq, Tk, holes, scale):
         assert dd["min_cos"] > 0.9999 and dd["max_rel"] < 1e-2, dd
 
 
+# The general scale's running max is a raw product: scores past the half range (inputs of +-60 at d = 128), a max that
+# jumps by more than 8 in log2 units on a middle and on the last tile, a negative scale, tiny scales, a causal prefix
+# and a cut last tile, in both types
+@pytest.mark.parametrize("dtype", [M.BF16, M.F16])
+@pytest.mark.parametrize("d,scale,mag,block", [(128, 128 ** -0.5, 60.0, 0), (64, 0.125, 3.0, 40), (128, -0.05, 1.0, 0),
+                                               (64, 1e-6, 1.0, 0), (64, 4.0, 1.0, 200)])
+def test_attention_general_scale_range(gpu, rng, dtype, d, scale, mag, block):
+    H, T = 2, 200
+    q_pad, k_pad = 256, 256
+    rnd, bits = (R.f16_round, M.f16_bits) if dtype == M.F16 else (R.bf16_round, M.bf16_bits)
+    q, k = (rnd((rng.standard_normal((1, H, T, d)) * mag).astype(np.float32)) for _ in range(2))
+    if mag == 60.0:
+        q, k = np.sign(q) * 60.0, np.sign(k) * 60.0
+        k[:, :, 70] = q[:, :, 5]    # 460 800 for query 5, far above its other scores
+        k[:, :, 199] = q[:, :, 90]
+    v = rnd(rng.standard_normal((1, H, T, d)).astype(np.float32))
+    Q, Kd = np.zeros((H, q_pad, d), np.float32), np.zeros((H, k_pad, d), np.float32)
+    Vt = np.zeros((H, d, k_pad), np.float32)
+    Q[:, :T], Kd[:, :T] = q[0], k[0]
+    Vt[:, :, M.vt_col(np.arange(T))] = v[0].transpose(0, 2, 1)
+    out = dev(np.zeros((T, H * d), np.uint16))
+    M.call("mk_attention", dev(bits(Q)).p, dev(bits(Kd)).p, dev(bits(Vt)).p, out.p, dtype, 1, H, H, d, T, q_pad, T, k_pad,
+           H * d, T * H * d, 0, block, scale, None, None)
+    M.sync()
+    got = fetch_bf16(out, (T, H, d))
+    s = np.einsum("hid,hjd->hij", q[0].astype(np.float64), k[0].astype(np.float64)) * scale
+    i, j = np.arange(T)[:, None], np.arange(T)[None]
+    s = np.where((i < block) & (j > i), -np.inf, s)
+    p = np.exp(s - s.max(-1, keepdims=True))
+    want = np.einsum("hij,hjd->ihd", p / p.sum(-1, keepdims=True), v[0].astype(np.float64))
+    # probabilities and outputs each rounded to 8 (bf16) bits; scores of up to 4.6e5 / 8 carry fp32 sums' 2^-23 of them
+    tol = 2 ** -7 + (2e-2 if mag == 60.0 else 0)
+    assert np.abs(got - want).max() <= tol * np.abs(want).max()
+
+
 # Launches of at most one tile a CU on 128-channel tiles run deep-staged (4 LDS stages for 128 x 128 tiles, 3 for
 # 256 x 128): K of 1 to 20 k steps covers the prologue, whole unrolled rounds and every remainder length.
 @pytest.mark.parametrize("K", [64, 128, 192, 256, 320, 448, 1280])
