@@ -135,7 +135,7 @@ mk_status mk_stream_create(void** s)
 mk_status mk_stream_destroy(void* s)
 {
     if (s) {
-        gemm_release_stream(s);
+        release_stream(s);
         MK_HIP(hipStreamDestroy(static_cast<hipStream_t>(s)));
     }
     return MK_OK;

@@ -66,9 +66,9 @@ double gemm_cost(const mk_gemm_args* a, uint32_t n, uint32_t cus);
 // MK_ERR_DEVICE when a stream-K launch on `stream` (all: on any stream of any device) gave up waiting for a partial
 // tile since the last check (the check clears it); called after synchronisations of that stream (all: of the device).
 mk_status gemm_take_error(const void* stream, bool all = false);
-// To be called before a stream is destroyed: waits for its last stream-K launch and frees that launch's workspace for
-// other streams (an event must not be asked after the stream it was recorded on is gone).
-void gemm_release_stream(const void* stream);
+// To be called before a stream is destroyed: waits for its last stream-K, split-K and group norm launches and frees their
+// workspaces for other streams (an event must not be asked after the stream it was recorded on is gone).
+void release_stream(const void* stream);
 
 // ---- ln_modulate over one or two problems in one launch (kernels.hip; the engine groups the two streams) ----
 struct LnArgs {
@@ -83,12 +83,15 @@ struct LnArgs {
 mk_status ln_modulate_group(const LnArgs* a, int count, uint32_t n, float eps, void* stream);
 
 // mk_layer_norm / mk_group_norm with the output in y_dtype (MK_BF16, or MK_F16: the input of a GEMM over half
-// weights), and fp32 -> IEEE half (nearest even) (kernels.hip)
+// weights) (kernels.hip)
 mk_status layer_norm_to(const float* x, uint32_t rows, uint32_t n, const float* g, const float* b, float eps, void* y,
                         uint32_t y_dtype, void* stream);
 mk_status group_norm_to(const float* x, uint32_t batch, uint32_t rows, uint32_t c, uint32_t groups, const float* g,
                         const float* b, float eps, void* y, uint32_t y_dtype, void* stream);
-mk_status f32_to_f16(const float* x, size_t n, void* y, void* stream);
+// hs to y_dtype (MK_BF16 or MK_F16) in y and x copied to out, n (a multiple of 4) floats each, 16-byte aligned
+mk_status convert_copy(const float* hs, const float* x, size_t n, void* y, uint32_t y_dtype, float* out, void* stream);
+// Before a stream is destroyed: waits for its last group norm and frees that call's scratch for other streams.
+void group_norm_release_stream(const void* stream);
 // mk_attention with the output in out_dtype (MK_BF16, or MK_F16: the input of a GEMM over half weights) (attention.hip)
 mk_status attention_to(const void* q, const void* k, const void* vt, void* out, uint32_t dtype, uint32_t batch,
                        uint32_t heads, uint32_t kv_heads, uint32_t d, uint32_t n_q, uint32_t q_pad, uint32_t n_k,

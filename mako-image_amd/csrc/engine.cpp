@@ -938,11 +938,9 @@ struct mk_engine {
             MK_TRY(gemm(B.ff2[0], hid.p, F, 0, nb * n, 1, hs, c, 0, MK_EPI_ADD, MK_F32, nullptr, 0, 0, 0, nullptr,
                         "gemm.ff2"));
         }
-        // proj_out + bias + the transformer's input
-        MK_HIP(hipMemcpyAsync(y, x, size_t(nb) * nc * 4, hipMemcpyDeviceToDevice, stream));
+        // proj_out + bias + the transformer's input, added into y: hs for the GEMM and x into y in one pass
         MK_TRY(timed("convert", 0, [&] {
-            return in_dt(proj_out) == MK_F16 ? f32_to_f16(hs, size_t(nb) * nc, xn_img.p, stream)
-                                             : mk_f32_to_bf16(hs, size_t(nb) * nc, xn_img.p, stream);
+            return convert_copy(hs, x, size_t(nb) * nc, xn_img.p, in_dt(proj_out), y, stream);
         }));
         MK_TRY(gemm(proj_out, xn_img.p, c, 0, nb * n, 1, y, c, 0, MK_EPI_ADD, MK_F32));
         return MK_OK;
@@ -1042,7 +1040,7 @@ mk_status mk_engine_destroy(mk_engine* e)
         (void)hipEventDestroy(e->ord_out);
     if (e->side)
         (void)hipStreamDestroy(e->side);
-    gemm_release_stream(e->stream);
+    release_stream(e->stream);
     (void)hipStreamDestroy(e->stream);
     delete e;
     return MK_OK;

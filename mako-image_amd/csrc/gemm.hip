@@ -1717,7 +1717,7 @@ mk_status sk_check(SkDevice& D, hipStream_t s, bool all)
 
 // Slabs of split-K launches: up to kSplitPool buffers of kSplitBytes a device, one a stream, so a stream's launches
 // follow each other on its own buffer and streams never share one. A stream beyond the pool takes the least recently
-// used buffer over after a device-wide wait; a destroyed stream's is given back by gemm_release_stream. (32 MB of slabs
+// used buffer over after a device-wide wait; a destroyed stream's is given back by release_stream. (32 MB of slabs
 // stay in the memory-side cache between the two kernels.) Locked with g_sk_mutex over both launches.
 constexpr size_t kSplitBytes = size_t(32) << 20, kSplitPool = 8;
 struct SplitWork {
@@ -2121,9 +2121,10 @@ mk_status prepare(const mk_gemm_args* a, GemmP& p, bool conv = false)
 
 } // namespace gemm_detail
 
-void gemm_release_stream(const void* stream)
+void release_stream(const void* stream)
 {
     using namespace gemm_detail;
+    group_norm_release_stream(stream);
     std::lock_guard<std::mutex> lock(g_sk_mutex);
     for (SkDevice& D : g_sk)
         for (auto& w : D.pool)

@@ -210,18 +210,21 @@ void launch_norm(uint32_t nvec, const float* x, uint32_t rows, uint32_t n, const
     norm_kernel<kRms, NV><<<cdiv(rows, 4), 256, 0, stream>>>(x, rows, n, g, b, w_offset, eps, y, f16);
 }
 
-// Group norm statistics (sdxl.cpp:425-437), two kernels: 16-row chunks of a sample, one workgroup each, sum x and
-// x^2 per channel in double over coalesced rows and reduce them per group through LDS (partials [batch][chunk][group]);
-// then one wave a (sample, group) adds its chunks and writes (mean, 1 / sqrt(var + eps)). (One workgroup a
-// (sample, group) walking the group's columns was a 181 us launch for 2 x 4096 x 640.)
+// Group norm statistics (sdxl.cpp:425-437), two kernels: 16-row chunks of a sample sum x and x^2 per channel in double
+// over coalesced rows and reduce them per group through LDS (partials [batch][chunk][group]); then one wave a (sample,
+// group) adds its chunks and writes (mean, 1 / sqrt(var + eps)). A workgroup takes a chunk's next `gp` groups, at most
+// 256 channels of them where a group has no more: one channel a thread, one memory wait, and enough workgroups to fill
+// the chip (one workgroup a chunk over all channels: 24.5 us for 2 x 1024 x 1280, 64 x 2 workgroups of 5 waits each;
+// 9.2 us in 6 parts).
 constexpr uint32_t kGnRows = 16;
 __global__ __launch_bounds__(256) void group_partial_kernel(const float* __restrict__ x, uint32_t rows, uint32_t c,
-                                                            uint32_t groups, double2* __restrict__ part)
+                                                            uint32_t groups, uint32_t gp, double2* __restrict__ part)
 {
-    __shared__ double ls[4096], lq[4096];
+    extern __shared__ double2 ls[]; // [gp c / groups]
     const uint32_t chunk = blockIdx.x, bi = blockIdx.y, r0 = chunk * kGnRows, r1 = min(rows, r0 + kGnRows);
-    const float* xb = x + uint64_t(bi) * rows * c;
-    for (uint32_t ch = threadIdx.x; ch < c; ch += 256) {
+    const uint32_t cg = c / groups, g0 = blockIdx.z * gp, ng = min(gp, groups - g0), nc = ng * cg;
+    const float* xb = x + uint64_t(bi) * rows * c + g0 * cg;
+    for (uint32_t ch = threadIdx.x; ch < nc; ch += 256) {
         // the chunk's rows all requested before the first add (one memory wait, not one a row), summed in row order
         float v[kGnRows];
 #pragma unroll
@@ -235,18 +238,26 @@ __global__ __launch_bounds__(256) void group_partial_kernel(const float* __restr
                 s += d;
                 q += d * d;
             }
-        ls[ch] = s;
-        lq[ch] = q;
+        ls[ch] = double2{s, q};
     }
     __syncthreads();
-    const uint32_t cg = c / groups;
-    for (uint32_t g = threadIdx.x; g < groups; g += 256) {
+    // 8 threads a group
+    const uint32_t l = threadIdx.x & 7;
+    for (uint32_t base = 0; base < ng; base += 32) {
+        const uint32_t g = base + (threadIdx.x >> 3);
         double s = 0.0, q = 0.0;
-        for (uint32_t i = 0; i < cg; ++i) {
-            s += ls[g * cg + i];
-            q += lq[g * cg + i];
+        if (g < ng)
+            for (uint32_t i = l; i < cg; i += 8) {
+                s += ls[g * cg + i].x;
+                q += ls[g * cg + i].y;
+            }
+#pragma unroll
+        for (int h = 4; h > 0; h >>= 1) {
+            s += __shfl_xor(s, h, 64);
+            q += __shfl_xor(q, h, 64);
         }
-        part[(uint64_t(bi) * gridDim.x + chunk) * groups + g] = double2{s, q};
+        if (l == 0 && g < ng)
+            part[(uint64_t(bi) * gridDim.x + chunk) * groups + g0 + g] = double2{s, q};
     }
 }
 
@@ -667,11 +678,6 @@ __global__ __launch_bounds__(256) void f2bf_kernel(const float* __restrict__ x, 
     for (uint64_t i = blockIdx.x * 256ull + threadIdx.x; i < n; i += uint64_t(gridDim.x) * 256)
         y[i] = f2bf_bits(x[i]);
 }
-__global__ __launch_bounds__(256) void f2h_kernel(const float* __restrict__ x, uint64_t n, uint16_t* __restrict__ y)
-{
-    for (uint64_t i = blockIdx.x * 256ull + threadIdx.x; i < n; i += uint64_t(gridDim.x) * 256)
-        y[i] = f2h_bits(x[i]);
-}
 __global__ __launch_bounds__(256) void bf2f_kernel(const uint16_t* __restrict__ x, uint64_t n, float* __restrict__ y)
 {
     for (uint64_t i = blockIdx.x * 256ull + threadIdx.x; i < n; i += uint64_t(gridDim.x) * 256)
@@ -959,7 +965,9 @@ static mk_status group_norm_run(const float* x, uint32_t batch, uint32_t rows, u
     const uint32_t chunks = cdiv(rows, kGnRows);
     double2* part = reinterpret_cast<double2*>(ws);
     float2* stats = reinterpret_cast<float2*>(ws + group_norm_part_bytes(batch, rows, groups));
-    group_partial_kernel<<<dim3(chunks, batch), 256, 0, s>>>(x, rows, c, groups, part);
+    const uint32_t cg = c / groups, gp = std::min(groups, std::max(1u, 256u / cg));
+    group_partial_kernel<<<dim3(chunks, batch, cdiv(groups, gp)), 256, sizeof(double2) * gp * cg, s>>>(x, rows, c, groups,
+                                                                                                     gp, part);
     group_final_kernel<<<dim3(groups, batch), 64, 0, s>>>(part, chunks, groups, double(rows) * double(c / groups), eps,
                                                           stats);
     const bool vec = c % 4 == 0 && uint64_t(rows) * c < (uint64_t(1) << 32) &&
@@ -976,13 +984,17 @@ static mk_status group_norm_run(const float* x, uint32_t batch, uint32_t rows, u
 }
 
 // mk_group_norm's partial sums: one buffer a device, grown (stream-ordered) when a call needs more and kept, so a
-// steady-state call allocates nothing. A call's stream first waits for the event of the buffer's previous user (any
-// stream), and records it after its own kernels: calls on different streams take turns on the buffer.
+// steady-state call allocates nothing. A call's stream first waits for the event of the buffer's previous user when that
+// was another stream, and records it after its own kernels: calls on different streams take turns on the buffer. A
+// stream that is about to be destroyed gives the buffer back (group_norm_release_stream): the event of a destroyed
+// stream must not be waited for.
 struct GnScratch {
     int dev = -1;
     char* p = nullptr;
     size_t bytes = 0;
     hipEvent_t last = nullptr;
+    hipStream_t owner = nullptr;
+    bool busy = false; // `owner` may still run the buffer's last user
 };
 static std::mutex g_gn_mutex;
 static std::vector<GnScratch> g_gn;
@@ -1016,9 +1028,11 @@ mk_status group_norm_to(const float* x, uint32_t batch, uint32_t rows, uint32_t 
         w = &g_gn.back();
         w->dev = dev;
         MK_HIP(hipEventCreateWithFlags(&w->last, hipEventDisableTiming));
-        MK_HIP(hipEventRecord(w->last, s));
     }
-    MK_HIP(hipStreamWaitEvent(s, w->last, 0));
+    if (w->busy && w->owner != s && hipStreamWaitEvent(s, w->last, 0) != hipSuccess) {
+        (void)hipGetLastError(); // its stream was destroyed elsewhere: wait for the whole device
+        MK_HIP(hipDeviceSynchronize());
+    }
     const size_t need = group_norm_scratch(batch, rows, groups);
     if (need > w->bytes) {
         if (w->p)
@@ -1031,7 +1045,19 @@ mk_status group_norm_to(const float* x, uint32_t batch, uint32_t rows, uint32_t 
     }
     const mk_status st = group_norm_run(x, batch, rows, c, groups, g, b, eps, y, w->p, s, y_dtype == MK_F16);
     MK_HIP(hipEventRecord(w->last, s));
+    w->owner = s;
+    w->busy = true;
     return st;
+}
+
+void group_norm_release_stream(const void* stream)
+{
+    std::lock_guard<std::mutex> lock(g_gn_mutex);
+    for (GnScratch& w : g_gn)
+        if (w.busy && w.owner == stream) {
+            (void)hipEventSynchronize(w.last);
+            w.busy = false;
+        }
 }
 
 mk_status layer_norm_to(const float* x, uint32_t rows, uint32_t n, const float* g, const float* b, float eps, void* y,
@@ -1047,14 +1073,33 @@ mk_status layer_norm_to(const float* x, uint32_t rows, uint32_t n, const float* 
     return MK_OK;
 }
 
-mk_status f32_to_f16(const float* x, size_t n, void* y, void* stream)
+// hs (fp32) to 16 bits in y and x copied to out (which may be x) in one pass, 4 values a thread: the copy and the
+// conversion apart took 5.6 + 5.7 us and a launch gap for 2 x 1024 x 1280
+template <bool F16>
+__global__ __launch_bounds__(256) void convert_copy_kernel(const float* __restrict__ hs, const float* x, uint64_t n4,
+                                                           uint16_t* __restrict__ y, float* out)
 {
-    if (!x || !y)
-        return fail(MK_ERR_ARG, "f32_to_f16: null pointer");
+    const uint64_t i = blockIdx.x * 256ull + threadIdx.x;
+    if (i >= n4)
+        return;
+    const f32x4 v = reinterpret_cast<const f32x4*>(hs)[i], u = reinterpret_cast<const f32x4*>(x)[i];
+    reinterpret_cast<u32x2*>(y)[i] = F16 ? u32x2{pack_f16x2(v[0], v[1]), pack_f16x2(v[2], v[3])}
+                                         : u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+    reinterpret_cast<f32x4*>(out)[i] = u;
+}
+
+mk_status convert_copy(const float* hs, const float* x, size_t n, void* y, uint32_t y_dtype, float* out, void* stream)
+{
+    if (!hs || !x || !y || !out || n % 4)
+        return fail(MK_ERR_ARG, "convert_copy: null pointer or a length that is not a multiple of 4");
     if (!n)
         return MK_OK;
-    f2h_kernel<<<grid_for(n), 256, 0, S(stream)>>>(x, n, static_cast<uint16_t*>(y));
-    MK_LAUNCH_CHECK("f32_to_f16");
+    const uint32_t grid = cdiv(n / 4, 256);
+    if (y_dtype == MK_F16)
+        convert_copy_kernel<true><<<grid, 256, 0, S(stream)>>>(hs, x, n / 4, static_cast<uint16_t*>(y), out);
+    else
+        convert_copy_kernel<false><<<grid, 256, 0, S(stream)>>>(hs, x, n / 4, static_cast<uint16_t*>(y), out);
+    MK_LAUNCH_CHECK("convert_copy");
     return MK_OK;
 }
 } // namespace mk

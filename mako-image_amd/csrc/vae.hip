@@ -627,7 +627,7 @@ struct mk_vae {
             if (b->p)
                 (void)hipFree(b->p);
         if (stream) {
-            gemm_release_stream(stream);
+            release_stream(stream);
             (void)hipStreamDestroy(stream);
         }
     }

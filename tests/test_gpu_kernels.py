@@ -1041,6 +1041,22 @@ def test_gemv_modulation(gpu, rng, rows, K, silu):
     assert maxrel(fetch(y, (rows, N)), want) < 1e-5
 
 
+# group norm: groups of one channel, of more channels than a workgroup's threads, more groups a workgroup than its
+# thread octets, groups that do not divide into whole workgroups; a cut last chunk of 16 rows
+@pytest.mark.parametrize("c,groups", [(40, 40), (96, 48), (1280, 32), (700, 7), (2048, 1), (608, 19)])
+@pytest.mark.parametrize("rows", [1, 50])
+def test_group_norm_partitions(gpu, rng, c, groups, rows):
+    x = (rng.standard_normal((2, rows, c)) * 2 + 0.5).astype(np.float32)
+    g, b = (1 + 0.1 * rng.standard_normal(c)).astype(np.float32), (0.1 * rng.standard_normal(c)).astype(np.float32)
+    y = dev(np.zeros(x.size, np.uint16))
+    M.call("mk_group_norm", dev(x).p, 2, rows, c, groups, dev(g).p, dev(b).p, 1e-2, y.p, None)
+    M.sync()
+    got = fetch_bf16(y, x.shape)
+    for i in range(2):
+        want = R.group_norm(x[i], g, b, groups, 1e-2)
+        assert np.abs(got[i] - want).max() <= 2 ** -8 * np.abs(want).max() + 1e-5  # one bf16 rounding
+
+
 # two rows share the one-row kernel's form for K in {2048, 3072, 4096}, three take the LDS-staged one: one output, a
 # workgroup's last pair cut
 @pytest.mark.parametrize("rows,K", [(2, 2048), (2, 4096), (3, 3072)])
