@@ -199,9 +199,9 @@ __device__ inline void epi_slice(const GemmP& p, const float* st, int ld, int to
     if constexpr (EK == EK_RMWUP) {
         // x + v (the convolution's ADD) goes to the four pixels (2 y + dy, 2 x + dx) of the nearest 2x grid, 16-bit;
         // the residual itself is not stored (its next reader is the upsampling). Tiles over the pixels only: every
-        // row of the slice is a pixel of image row y.
+        // row of the slice is a pixel of image row y; else the row's pixel by an integer division, ring rows left out.
         const float* c = static_cast<const float*>(p.c) + ch;
-        const uint32_t pw = p.conv_pw, y = uint32_t(tok0) / pw - 1, ld2 = p.norm_ld;
+        const uint32_t pw = p.conv_pw, gh = p.M / pw, gy0 = uint32_t(tok0) / pw, ld2 = p.norm_ld;
         uint16_t* up = p.norm_out + ch;
         f32x4 xs[NI];
 #pragma unroll
@@ -213,9 +213,9 @@ __device__ inline void epi_slice(const GemmP& p, const float* st, int ld, int to
             for (int i = 0; i < NI; ++i) {
                 const int t = tok0 + r0 + RPI * i;
                 const f32x4& x = xs[i];
-                if (t < int(p.M)) {
-                    const uint32_t xx = uint32_t(t) - (y + 1) * pw - 1;
-                    const uint64_t r = p.up_slack + uint64_t(2 * y + 1) * p.up_pw + 2 * xx + 1;
+                const uint32_t gy = p.conv_w ? gy0 : uint32_t(t) / pw, gx = uint32_t(t) - gy * pw;
+                if (t < int(p.M) && (p.conv_w || (gy >= 1 && gy + 1 < gh && gx >= 1 && gx + 1 < pw))) {
+                    const uint64_t r = p.up_slack + uint64_t(2 * gy - 1) * p.up_pw + 2 * gx - 1;
                     const u32x2 o{pack16<H>(x[0] + v[i][0], x[1] + v[i][1]), pack16<H>(x[2] + v[i][2], x[3] + v[i][3])};
                     *reinterpret_cast<u32x2*>(up + r * ld2) = o;
                     *reinterpret_cast<u32x2*>(up + (r + 1) * ld2) = o;
@@ -2451,10 +2451,10 @@ mk_status conv3x3_run(const mk_conv_args* a, uint32_t lda, bool dense, const Con
                         : (a->y_dtype != MK_F16 || a->epilogue != MK_EPI_STORE))))
         return fail(MK_ERR_ARG, std::string(who) + ": the norm epilogues need 96 or 192 output channels and a gain, "
                                                    "and either an f16 store or an fp32 output plus a normed one");
-    if (up && (nm || dense || !up->out || a->epilogue != MK_EPI_ADD || a->n % 192 || a->width % 256 || up->ld < a->n ||
+    if (up && (nm || dense || !up->out || a->epilogue != MK_EPI_ADD || a->n % 192 || up->ld < a->n ||
                up->ld % 4 || a->h > (1u << 14) || a->width > (1u << 14)))
-        return fail(MK_ERR_ARG, std::string(who) + ": the 2x-grid epilogue needs an ADD over 192-channel multiples, "
-                                                   "an image width of a multiple of 256 and no norm epilogue");
+        return fail(MK_ERR_ARG, std::string(who) + ": the 2x-grid epilogue needs an ADD over 192-channel multiples "
+                                                   "and no norm epilogue");
     const uint64_t pw = uint64_t(a->width) + 2, rows = (uint64_t(a->h) + 2) * pw;
     if (rows >= (1u << 31) || (256 + 2 * pw + 2) * lda * 2 >= (uint64_t(1) << 32) || a->ldy < a->n)
         return fail(MK_ERR_ARG, std::string(who) + ": image too large or ldy < n");
@@ -2489,14 +2489,14 @@ mk_status conv3x3_run(const mk_conv_args* a, uint32_t lda, bool dense, const Con
         plan.bm = a->n == 96 ? 128 : 256;
         plan.bn = a->n;
     }
-    if (up) { // 256 x 192 tiles over the pixels: a tile's rows lie in one image row
+    if (up) {
         plan.bm = 256;
         plan.bn = 192;
     }
     if (a->width % plan.bm == 0) {
         p.conv_w = a->width;
         p.conv_pix = gp.M;
-    } else if (!nm) {
+    } else if (!nm && !up) {
         plan = gemm_plan(&g, 1, uint32_t(cus > 0 ? cus : 1), true);
     }
     plan.sk = false;

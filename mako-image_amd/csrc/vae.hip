@@ -937,7 +937,8 @@ struct mk_vae {
     mk_status attention(GridDims g, float* xp)
     {
         const uint32_t c = qkv.co, cp = qkv.cip();
-        const uint64_t n = uint64_t(g.h) * g.w, np = (n + 63) / 64 * 64;
+        // whole 256-wide tiles once the padding is small (a chunk's scores over 15808 pixels: 79 us on 64-wide tiles, 64)
+        const uint64_t n = uint64_t(g.h) * g.w, np = round_up(n, n >= 4096 ? 256 : 64);
         // q2 [np][2 cp] = [Q | Q], k2 [np][2 cp] = [K_hi | K_lo], vt2 [2 cp][np] = [V^T_hi ; V^T_lo] (halves); kf the
         // fp32 projections (K [np][cp], then V^T [cp][np]); the normed pixels [np][cp] (rows past n zero)
         MK_TRY(ensure(qb, np * cp * 4));
@@ -1084,11 +1085,13 @@ struct mk_vae {
         for (int i = 0; i < 4; ++i) {
             Up& u = ups[i];
             // the last res block's conv2 can write the nearest-2x grid the upsampling conv reads (into sc, since its
-            // input may be a): whole 192-channel tiles over the pixels of one image row each
+            // input may be a) from 256 x 192 tiles: where those cover whole image rows, and at other widths where
+            // they are about two rounds of 256 compute units (832 x 1216: the two convolutions 171 -> 214 and 216 -> 288 us,
+            // vae_up's 76 + 173 us gone); the smaller levels keep the convolution's own tiles and vae_up
             const Res& rl = u.res[2];
             const bool up_fused = u.up && !rl.shortcut && !rl.c2.dense && rl.c2.co % 192 == 0 &&
                                   rl.c2.cop() == rl.c2.co && u.cout == rl.c2.co && u.conv.cip() == rl.c2.co &&
-                                  g.w % 256 == 0;
+                                  (g.w % 256 == 0 || g.grid_rows() / 256 * (rl.c2.co / 192) >= 500);
             uint16_t* const upbuf = up_fused ? ns : na;
             for (int j = 0; j < 3; ++j) {
                 const Res& r = u.res[j];

@@ -154,6 +154,45 @@ def test_vae_decode_matches_oracle(gpu, base, h, w):
     assert np.array_equal(vae.decode(tokens, h, w), got)
 
 
+def test_vae_decode_of_a_width_no_tile_divides(gpu):
+    # 45 x 46 tokens: the 192-channel level (360 x 368 pixels) writes the 2x grid from tiles over the padded rows, and
+    # the mid block's 8280 pixels are padded to whole 256-wide tiles; against the decoder in torch's fp32, its
+    # convolutions' operands rounded to half as the kernels' are
+    base, h, w = 96, 45, 46
+    ref = R.Vae(base, seed=5, mean=MEAN, std=STD)
+    vae = M.Vae(base, mean=MEAN, std=STD)
+    vae.init_random(5)
+    tokens = np.random.default_rng(3).standard_normal((h * w, 64)).astype(np.float32)
+    t = {n: torch.from_numpy(a) for n, a in ref.tensors()}
+    half = lambda x: x.half().float()  # noqa: E731
+
+    def conv(x, name):
+        wt = t[name + ".weight"]
+        return F.conv2d(half(x), half(wt), t[name + ".bias"], padding=wt.shape[-1] // 2)
+
+    def rms(x, g, act=F.silu):
+        return act(F.normalize(x, dim=1, eps=1e-12) * x.shape[1] ** 0.5 * t[g][None, :, None, None])
+
+    def res(x, p):
+        y = conv(rms(conv(rms(x, p + ".norm1.gamma"), p + ".conv1"), p + ".norm2.gamma"), p + ".conv2")
+        return y + (conv(x, p + ".conv_shortcut") if p + ".conv_shortcut.weight" in t else x)
+
+    lat = torch.from_numpy(tokens).reshape(h, w, 16, 2, 2).permute(2, 0, 3, 1, 4).reshape(1, 16, 2 * h, 2 * w)
+    x = lat * torch.from_numpy(STD)[None, :, None, None] + torch.from_numpy(MEAN)[None, :, None, None]
+    x = res(conv(conv(x, "post_quant_conv"), "decoder.conv_in"), "decoder.mid_block.resnets.0")
+    a = "decoder.mid_block.attentions.0."
+    q, k, v = conv(rms(x, a + "norm.gamma", lambda y: y), a + "to_qkv").flatten(2)[0].T.chunk(3, 1)
+    x = x + conv((torch.softmax(half(q) @ k.T / k.shape[1] ** 0.5, -1) @ v).T.reshape(x.shape), a + "proj")
+    x = res(x, "decoder.mid_block.resnets.1")
+    for i in range(4):
+        for j in range(3):
+            x = res(x, f"decoder.up_blocks.{i}.resnets.{j}")
+        if i < 3:
+            x = conv(F.interpolate(x, scale_factor=2, mode="nearest"), f"decoder.up_blocks.{i}.upsamplers.0.resample.1")
+    want = conv(rms(x, "decoder.norm_out.gamma"), "decoder.conv_out")[0].permute(1, 2, 0).clamp(-1, 1).numpy()
+    within(vae.decode(tokens, h, w)[..., :3], want, 3)
+
+
 def test_vae_mid_attention_over_256_pixels(gpu):
     # 8 x 8 tokens: 256 pixels in the mid block, whose one-head attention (scores, softmax, P V) runs over all of them;
     # the mid block's output against the oracle's exact softmax (the smaller decodes above check the whole path).
