@@ -59,8 +59,9 @@ struct GemmPlan {
     double cost;     // estimated duration in units of one k step of a 256 x 256 tile
 };
 // The plan of a launch of n grouped problems (equal N, K, weight type, epilogue kind) on `cus` compute units;
-// `conv`: a 3 x 3 convolution (256-token tiles only).
-GemmPlan gemm_plan(const mk_gemm_args* a, uint32_t n, uint32_t cus, bool conv = false);
+// `conv`: a 3 x 3 convolution; `by_row`: its input channels are a multiple of 32 (conv_kernel's 96- and 192-channel
+// tiles).
+GemmPlan gemm_plan(const mk_gemm_args* a, uint32_t n, uint32_t cus, bool conv = false, bool by_row = false);
 // Its estimated duration in units of one 256-channel k step.
 double gemm_cost(const mk_gemm_args* a, uint32_t n, uint32_t cus);
 // MK_ERR_DEVICE when a stream-K launch on `stream` (all: on any stream of any device) gave up waiting for a partial

@@ -51,7 +51,7 @@ struct GemmP {
     HeadsP hp;
     // 3 x 3 convolution (EK_CONV): the padded grid's row width w + 2, k tiles a tap (channels / 64), and
     // ceil(2^16 / conv_tpt) for the tap index by multiply-shift; with EK_CONVQ conv_tpt counts 8-channel chunks
-    uint32_t conv_pw, conv_tpt, conv_inv;
+    uint32_t conv_pw, conv_tpt, conv_inv, conv_c; // (conv_c: input channels)
     // With conv_w (the image width, a multiple of BM) the tiles cover the conv_pix = h w pixels only, BM of one image
     // row each (tile tm: pixel tm BM, grid row (y + 1) pw + x + 1), so no tile is spent on ring rows and the launch
     // holds whole rounds where h w does; the ring's output rows are then not written.
@@ -1454,6 +1454,222 @@ __global__ __launch_bounds__(64 * NW, BM == 128 && !(EK & EK_DEEP) ? 2 : 1) __at
     gemm_tile<BM, BN, kF8, EK, NW>(p, z, tm, tn, 0, int(p.K) / BK, smem, nullptr, -1);
 }
 
+// 3 x 3 convolutions with tiles of 96 (4 waves, 128 pixels) or 192 (8 waves, 256 pixels) output channels, a wave 96
+// channels of 32 or 64 pixels on v_mfma_f32_16x16x32_f16, over input channels in multiples of 32. A k step is one row of
+// taps (dy) and 32 channels, 96 deep: its three taps read the same BM + 2 input rows, which come in once, not once a
+// tap as in gemm_tile's 64-deep steps: 27 KB a step for 128 x 96 instead of 28 KB for 64 deep, 53 instead of 57 for 256 x
+// 192, so three stages fit (two workgroups a CU for the 96-channel tiles) and a step's direct loads have two steps to
+// land. LDS rows: the weights' 192 bytes [dx][32 channels], the input's 64; 16-byte chunks swizzled by (row >> 2) & 3
+// within each 64 bytes, so 16 rows at one chunk cover all banks. One barrier a step, between its second and third tap:
+// behind it the third tap's products read the next step's first fragments and refill this step's stage. The 96-channel
+// tiles take 256 pixels (64 a wave: 10 fragment reads for 24 products instead of 8 for 12, the LDS bound of 128 pixels)
+// with two stages where that leaves two rounds of them. Measured at 1024 x 1024, 96 channels, on one box: norm epilogue
+// 274 -> 226 us (280 on 128-pixel tiles), adding and norming the fp32 residual 334 -> 270 (HBM: 1.2 GB), from 192
+// channels 466 -> 430; at 512 x 512, 192 channels, adding and norming 292 -> 269, norm alone 189 -> 191. The fp32
+// residual and the 192-channel tiles' uncovered epilogue (one workgroup a CU) bound what is left.
+template <int BN, int BM, int EKE>
+__global__ __launch_bounds__(BN * 8 / 3, BN == 96 ? 2 : 1) __attribute__((amdgpu_waves_per_eu(2, 2))) void conv_kernel(
+    GemmG G)
+{
+    constexpr int NW = BN / 24, WCH = BN / 96, WM = BM / (NW / WCH), NSTG = BN == 96 && BM == 256 ? 2 : 3;
+    constexpr int CB = 6, TB = WM / 16, NS = WM / 32, LDW = 96 + 4;
+    constexpr int WI = BN * 12 / 64, AI = BM / 16, TAIL = WI + AI; // loads of the weights, of the input's first BM rows,
+    constexpr int ND = (TAIL + NW) / NW;                           // then one of its last 16; loads a wave
+    constexpr int WB = BN * 192, SB = WB + (BM + 2) * 64;          // bytes: the weights, a stage
+    static_assert(NSTG * SB * (BN == 96 ? 2 : 1) <= 160 * 1024, "the stages fit the LDS");
+    // a stage is an object of its own, so the reads of one do not wait for the loads into another
+    __shared__ __attribute__((aligned(16))) uint16_t s0[SB / 2], s1[SB / 2],
+        s2[NSTG == 3 ? SB / 2 : 8];
+    auto stage = [&](int i) { return i == 0 ? s0 : i == 1 ? s1 : s2; };
+    uint32_t z, tm, tn;
+    const GemmP& p = locate(G, xcd_order(blockIdx.x, gridDim.x), z, tm, tn);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wn = WCH == 2 ? wave & 1 : 0, wm = WCH == 2 ? wave >> 1 : wave, r16 = lane & 15, g4 = lane >> 4;
+    const int n0 = int(tn) * BN, pw = int(p.conv_pw), lda = int(p.lda), c = int(p.conv_c), nc = c / 32;
+    int m0 = int(tm) * BM;
+    if (p.conv_w) {
+        const int y = m0 / int(p.conv_w), x = m0 - y * int(p.conv_w);
+        m0 = (y + 1) * pw + x + 1;
+    }
+    const int rows = min(int(p.M) - m0, BM); // (rows past M read the last row's neighbourhood and are not stored)
+    const BufRes rsA = buf_res(p.a + int64_t(m0) * lda, uint32_t((rows + 2 * int64_t(pw) + 2) * lda * 2));
+    const BufRes rsW = buf_res(static_cast<const uint16_t*>(p.w) + int64_t(n0) * p.K, uint32_t(BN) * p.K * 2);
+    // a wave's load i: slot i NW + wave; slots from TAIL on load the input's last 16 rows (14 of them again)
+    uint32_t off[ND];
+#pragma unroll
+    for (int i = 0; i < ND; ++i) {
+        const int q = i * NW + wave;
+        if (q < WI) {
+            const int P = q * 64 + lane, row = P / 12, sl = P - row * 12, g = (sl & 3) ^ ((row >> 2) & 3);
+            off[i] = uint32_t(row * int(p.K) + (sl >> 2) * c + g * 8) * 2;
+        } else {
+            const int j = (q < TAIL ? (q - WI) * 16 : BM - 14) + (lane >> 2), g = (lane & 3) ^ ((j >> 2) & 3);
+            off[i] = uint32_t(min(j, rows + 1) * lda + g * 8) * 2;
+        }
+    }
+    // LDS element offset of the last round's load (the others': slot * 512, the input behind the weights)
+    const int last_to = (ND - 1) * NW + wave < TAIL ? ((ND - 1) * NW + wave) * 512 : WB / 2 + (BM - 14) * 32;
+    // the step the next loads are of: tap row ld_y, channel chunk ld_c (past the last step: the last one again)
+    int ld_y = 0, ld_c = 0;
+    auto dma1 = [&](auto st_c, int i) {
+        constexpr int st = decltype(st_c)::value;
+        const uint32_t kw = uint32_t(ld_y * 3 * c + ld_c * 32) * 2, ka = uint32_t(ld_y * pw * lda + ld_c * 32) * 2;
+        const int q = i * NW + wave;
+        lds_void* to = (lds_void*)&stage(st)[i == ND - 1 ? last_to : q * 512];
+        if (i * NW + NW <= WI)
+            buf_load_lds16(rsW, to, off[i], kw);
+        else if (i * NW >= WI)
+            buf_load_lds16(rsA, to, off[i], ka);
+        else // the round that holds both
+            buf_load_lds16(q < WI ? rsW : rsA, to, off[i], q < WI ? kw : ka);
+    };
+    auto next_step = [&] {
+        if (ld_c + 1 < nc)
+            ++ld_c;
+        else if (ld_y < 2) {
+            ld_c = 0;
+            ++ld_y;
+        }
+    };
+    auto issue = [&](auto st_c) {
+#pragma unroll
+        for (int i = 0; i < ND; ++i)
+            dma1(st_c, i);
+        next_step();
+    };
+    f32x4 acc[CB][TB];
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb)
+            acc[cb][tb] = f32x4{};
+    // fragments: weight rows (wn 96 + 16 cb + r16), chunk 4 dx + g4; input rows (wm WM + 16 tb + r16 + dx), chunk g4
+    const int wbase = (wn * 96 + r16) * 96 + ((g4 ^ (r16 >> 2)) << 3);
+    int abase[3];
+#pragma unroll
+    for (int dx = 0; dx < 3; ++dx)
+        abase[dx] = WB / 2 + (wm * WM + r16 + dx) * 32 + ((g4 ^ (((r16 + dx) >> 2) & 3)) << 3);
+    f16x8v wf[CB], af[3][TB];
+    auto rdw = [&](int st, int dx, int cb) {
+        wf[cb] = *reinterpret_cast<const f16x8v*>(&stage(st)[wbase + cb * 16 * 96 + dx * 32]);
+    };
+    auto rda = [&](int st, int dx, int tb) {
+        af[dx][tb] = *reinterpret_cast<const f16x8v*>(&stage(st)[abase[dx] + tb * 16 * 32]);
+    };
+    // tap DX's products; the next fragments (tap NDX of stage NST) are read behind the products that free their
+    // registers, and with LD the loads of NSTG steps on go into stage LST
+    auto tap = [&](auto dx_c, auto nst_c, auto ndx_c, auto ld_c2, auto lst_c) {
+        constexpr int DX = decltype(dx_c)::value, NST = decltype(nst_c)::value, NDX = decltype(ndx_c)::value;
+        constexpr bool LD = decltype(ld_c2)::value;
+#pragma unroll
+        for (int i = 0; i < CB * TB; ++i) {
+            const int cb = i / TB, tb = i % TB;
+            acc[cb][tb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf[cb], af[DX][tb], acc[cb][tb], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            if (cb == 0) {
+                rda(NST, NDX, tb);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (tb == TB - 1) {
+                rdw(NST, NDX, cb);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (LD && i < ND) {
+                dma1(lst_c, i);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if constexpr (LD)
+            next_step();
+    };
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
+    auto sync = [&](auto vm_c) {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(waitcnt_bits(decltype(vm_c)::value, 0));
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto step = [&](auto st_c) {
+        constexpr int st = decltype(st_c)::value;
+        const std::integral_constant<int, (st + 1) % NSTG> nst_c;
+        tap(I0{}, st_c, I1{}, std::false_type{}, st_c);
+        tap(I1{}, st_c, I2{}, std::false_type{}, st_c);
+        // the next step landed (a third stage's loads may be in flight); every wave done reading this one's stage
+        sync(std::integral_constant<int, (NSTG - 2) * ND>{});
+        tap(I2{}, nst_c, I0{}, std::true_type{}, st_c);
+    };
+    issue(I0{});
+    issue(I1{});
+    if constexpr (NSTG == 3)
+        issue(I2{});
+    sync(std::integral_constant<int, (NSTG - 1) * ND>{});
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb)
+        rdw(0, 0, cb);
+#pragma unroll
+    for (int tb = 0; tb < TB; ++tb)
+        rda(0, 0, tb);
+    if constexpr (NSTG == 3) {
+        for (int k = 0; k < nc; ++k) { // 3 nc steps
+            step(I0{});
+            step(I1{});
+            step(I2{});
+        }
+    } else {
+        int k = 0;
+        for (; k + 1 < 3 * nc; k += 2) {
+            step(I0{});
+            step(I1{});
+        }
+        if (k < 3 * nc)
+            step(I0{});
+    }
+    __builtin_amdgcn_s_waitcnt(0); // the last (unused) loads land before the LDS is reused
+    __syncthreads();
+    // epilogue: each wave stages 32 pixels x 96 channels (fp32) in a region of its own
+    static_assert(NW / 2 * 32 * LDW * 4 <= SB && 2 * NW * 32 * 4 <= SB, "half the waves' staging fits a stage");
+    float* st = reinterpret_cast<float*>(wave < NW / 2 ? s0 : s1) + (wave % (NW / 2)) * 32 * LDW;
+    float* xch = reinterpret_cast<float*>(NSTG == 3 ? s2 : s1); // (192 channels only)
+    EpiCh kch[3];
+    if constexpr (EKE != EK_NORM && EKE != EK_RMWN)
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+            kch[j] = epi_channels(p, n0 + wn * 96 + 32 * j + 4 * (lane % 8));
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                *reinterpret_cast<f32x4*>(st + (16 * h + r16) * LDW + cb * 16 + 4 * g4) = acc[cb][2 * s + h];
+        const int tok = m0 + wm * WM + s * 32;
+        if constexpr (EKE == EK_NORM || EKE == EK_RMWN)
+            epi_norm_silu<EKE, WCH == 2, true>(p, st, LDW, tok, wn * 96, lane, xch + (s & 1) * NW * 32, wave);
+        else
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+                epi_slice<EKE, 32>(p, st + 32 * j, LDW, tok, n0 + wn * 96 + 32 * j, lane, 0, kch[j]);
+    }
+}
+
+template <int BN, int EKE> mk_status launch_conv(GemmP& p, int bm, hipStream_t s)
+{
+    GemmG G{};
+    p.tiles_m = p.conv_w ? p.conv_pix / bm : cdiv(p.M, bm);
+    p.tiles_n = p.N / BN;
+    G.g[0] = p;
+    G.tiles0 = p.tiles_m * p.tiles_n;
+    if (BN == 96 && bm == 128)
+        conv_kernel<BN, BN == 96 ? 128 : 256, EKE><<<G.tiles0, BN * 8 / 3, 0, s>>>(G);
+    else
+        conv_kernel<BN, 256, EKE><<<G.tiles0, BN * 8 / 3, 0, s>>>(G);
+    MK_HIP(hipGetLastError());
+    return MK_OK;
+}
+
 // Split-K for launches of few tiles (a prompt's rows, a small image): `splits` workgroups share a tile's k steps and
 // store their fp32 partial tiles, unscaled, one slab of all rows a split; gemm_reduce_kernel then adds the slabs in
 // order and runs the epilogue. G holds the partials' C (the slab; its row stride N, no scale, bias or gate).
@@ -2162,7 +2378,7 @@ mk_status gemm_take_error(const void* stream, bool all)
 // a tile is long (K of 6144 or more; measured, the partials' exchange costs about 24 k steps of a tile, more than the
 // balance saves on shorter tiles): the whole waves go round robin, the rest is split by k steps (at least 4 a
 // workgroup).
-GemmPlan gemm_plan(const mk_gemm_args* a, uint32_t n, uint32_t cus, bool conv)
+GemmPlan gemm_plan(const mk_gemm_args* a, uint32_t n, uint32_t cus, bool conv, bool by_row)
 {
     const uint64_t kt = a[0].K / gemm_detail::BK;
     const uint32_t N = a[0].N;
@@ -2219,7 +2435,7 @@ GemmPlan gemm_plan(const mk_gemm_args* a, uint32_t n, uint32_t cus, bool conv)
     consider(256, 128, 0.66);
     if (conv)
         consider(256, 192, 0.78);
-    if (conv && N % 64) // 96 output channels (and odd multiples of 96) take 128 x 96 tiles, nothing else
+    if (conv && (N % 64 || by_row)) // 96 output channels (and odd multiples of 96) take 128 x 96 tiles, nothing else
         consider(128, 96, 0.5);
     if (narrow_ok)
         consider(256, 64, 0.62);
@@ -2478,13 +2694,15 @@ mk_status conv3x3_run(const mk_conv_args* a, uint32_t lda, bool dense, const Con
     p.conv_pw = uint32_t(pw);
     p.conv_tpt = dense ? a->c / 8 : a->c / 64;
     p.conv_inv = (65536u + p.conv_tpt - 1) / p.conv_tpt;
+    p.conv_c = a->c;
+    const bool by_row = a->c % 32 == 0; // 96- and 192-channel tiles: conv_kernel
     int cus = 0, dev = 0;
     MK_HIP(hipGetDevice(&dev));
     MK_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
     // tiles over the pixels when the plan for h w rows has a tile height dividing w, else over the padded rows
     mk_gemm_args gp = g;
     gp.M = a->h * a->width;
-    GemmPlan plan = gemm_plan(&gp, 1, uint32_t(cus > 0 ? cus : 1), true);
+    GemmPlan plan = gemm_plan(&gp, 1, uint32_t(cus > 0 ? cus : 1), true, by_row);
     if (nm) { // the norm epilogues' tiles span the row: 128 x 96 or 256 x 192
         plan.bm = a->n == 96 ? 128 : 256;
         plan.bn = a->n;
@@ -2493,11 +2711,18 @@ mk_status conv3x3_run(const mk_conv_args* a, uint32_t lda, bool dense, const Con
         plan.bm = 256;
         plan.bn = 192;
     }
+    // 96-channel tiles of 256 pixels (conv_kernel) from two rounds of them on, two a CU (one round and less of 128-pixel
+    // tiles keep more workgroups in flight: 128 x 128 pixels of 384 channels are 512 of them, 56 us)
+    const bool tall = by_row && plan.bn == 96 && uint64_t(gp.M) * (a->n / 96) >= uint64_t(256) * 4 * uint64_t(cus);
+    if (tall)
+        plan.bm = 256;
     if (a->width % plan.bm == 0) {
         p.conv_w = a->width;
         p.conv_pix = gp.M;
     } else if (!nm && !up) {
-        plan = gemm_plan(&g, 1, uint32_t(cus > 0 ? cus : 1), true);
+        plan = gemm_plan(&g, 1, uint32_t(cus > 0 ? cus : 1), true, by_row);
+        if (tall && plan.bn == 96)
+            plan.bm = 256;
     }
     plan.sk = false;
     hipStream_t s = static_cast<hipStream_t>(stream);
@@ -2508,26 +2733,28 @@ mk_status conv3x3_run(const mk_conv_args* a, uint32_t lda, bool dense, const Con
         p.norm_ld = up->ld;
         p.up_pw = 2 * a->width + 2;
         p.up_slack = 2 * a->width + 3;
-        return launch<256, 192, false, EK_RMWUP | C, 8>(&p, 1, plan, s);
+        return launch_conv<192, EK_RMWUP>(p, plan.bm, s); // (c a multiple of 64)
     }
     if (nm) {
         p.norm_g = nm->g;
         p.norm_out = nm->out;
         p.norm_ld = nm->ld;
         p.norm_only = nm->out && nm->skip_y ? 1u : 0u;
-        if (a->n == 192) {
-            if (nm->out)
-                return dense ? launch<256, 192, false, EK_RMWN | Q, 8>(&p, 1, plan, s)
-                             : launch<256, 192, false, EK_RMWN | C, 8>(&p, 1, plan, s);
-            return dense ? launch<256, 192, false, EK_NORM | Q, 8>(&p, 1, plan, s)
-                         : launch<256, 192, false, EK_NORM | C, 8>(&p, 1, plan, s);
-        }
-        if (nm->out)
-            return dense ? launch<128, 96, false, EK_RMWN | Q, 4>(&p, 1, plan, s)
-                         : launch<128, 96, false, EK_RMWN | C, 4>(&p, 1, plan, s);
-        return dense ? launch<128, 96, false, EK_NORM | Q, 4>(&p, 1, plan, s)
-                     : launch<128, 96, false, EK_NORM | C, 4>(&p, 1, plan, s);
+        if (by_row && a->n == 192)
+            return nm->out ? launch_conv<192, EK_RMWN>(p, plan.bm, s) : launch_conv<192, EK_NORM>(p, plan.bm, s);
+        if (by_row)
+            return nm->out ? launch_conv<96, EK_RMWN>(p, plan.bm, s) : launch_conv<96, EK_NORM>(p, plan.bm, s);
+        // (channels that are not a multiple of 32 are dense)
+        if (a->n == 192)
+            return nm->out ? launch<256, 192, false, EK_RMWN | Q, 8>(&p, 1, plan, s)
+                           : launch<256, 192, false, EK_NORM | Q, 8>(&p, 1, plan, s);
+        return nm->out ? launch<128, 96, false, EK_RMWN | Q, 4>(&p, 1, plan, s)
+                       : launch<128, 96, false, EK_NORM | Q, 4>(&p, 1, plan, s);
     }
+    if (by_row && plan.bn == 96)
+        return add ? launch_conv<96, EK_RMW>(p, plan.bm, s) : launch_conv<96, EK_STORE>(p, plan.bm, s);
+    if (by_row && plan.bn == 192)
+        return add ? launch_conv<192, EK_RMW>(p, plan.bm, s) : launch_conv<192, EK_STORE>(p, plan.bm, s);
     // (the tile shapes a convolution's plan may take, each with the implicit-GEMM flags of its K layout)
     auto go = [&](auto f) -> mk_status {
         if (plan.bn == 96)
@@ -2545,7 +2772,9 @@ mk_status conv3x3_run(const mk_conv_args* a, uint32_t lda, bool dense, const Con
     auto shape = [&](auto sel, auto flags) -> mk_status {
         constexpr int i = decltype(sel)::value, F = decltype(flags)::value;
         constexpr int EK = (i % 2 ? EK_STORE : EK_RMW) | F;
-        if constexpr (i / 2 == 0)
+        if constexpr (F == C && (i / 2 == 0 || i / 2 == 3))
+            return fail(MK_ERR_UNSUPPORTED, "conv3x3: 96- and 192-channel tiles by rows only"); // (conv_kernel took it)
+        else if constexpr (i / 2 == 0)
             return launch<128, 96, false, EK, 4>(&p, 1, plan, s);
         else if constexpr (i / 2 == 1)
             return launch<128, 128, false, EK, 4>(&p, 1, plan, s);
