@@ -129,7 +129,9 @@ typedef struct mk_gemm_args {
 } mk_gemm_args;
 
 /* proj (the reference's GEMM, engine.cpp:768 / qwen_image.cpp:196-288): C = A W^T with the fused epilogue.
- * K % 64 == 0, N % 64 == 0. */
+ * K % 64 == 0, N % 64 == 0. Launches of fewer than 1024 rows may split their k steps over workgroups into fp32 slabs of the
+ * library's (at most 8 x 32 MB a device, one a stream; whole tiles when the stream is being captured): the sums then run
+ * in another, fixed order than a larger launch's. */
 mk_status mk_gemm(const mk_gemm_args* a, void* stream);
 /* count (1 or 2) GEMMs of equal N, K, weight dtype and epilogue kind in one launch: the dual-stream blocks' image and
  * text projections, whose separate launches would leave most of the chip idle on the text's few tiles. Each problem

@@ -219,11 +219,12 @@ __global__ __launch_bounds__(64 * NW, 2) __attribute__((amdgpu_waves_per_eu(2, 2
     // loads provably touch different buffers and the reads wait for nothing but themselves), the softmax work in the
     // matrix core's shadow. The tile's 32 fragment reads stream LA ahead of the MFMAs that use them, in a fixed order
     // (fenced). The scores arrive as S - m, so each half's probabilities are computed speculatively, before its row max
-    // is known: P = 2^(c (S - m)) is what the tile needs whenever no score exceeds m by more than kLazy in log2 units. The exponentials, conversions and row sums of half a then
-    // run in chunks between the S^T MFMAs of half b, those of half b between the P V MFMAs of half a, and the lane's
-    // part of the row sum only decides afterwards whether a half is redone against a new m (the first half of the
-    // pass, and the rare tiles whose max jumps: a score more than kLazy above m puts that sum above 2^kLazy). EDGE
-    // tiles (ragged key end, causal diagonal, a masked key range) mask scores in the chunks.
+    // is known: P = 2^(c (S - m)) is what the tile needs whenever no score exceeds m by more than kLazy in log2 units.
+    // The exponentials, conversions and row sums of half a then run in chunks between the S^T MFMAs of half b, those of
+    // half b between the P V MFMAs of half a, and the lane's part of the row sum only decides afterwards whether a half
+    // is redone against a new m (the first half of the pass, and the rare tiles whose max jumps: a score more than kLazy
+    // above m puts that sum above 2^kLazy). EDGE tiles (ragged key end, causal diagonal) mask scores in the chunks; a
+    // masked key range is masked by the product that subtracts m.
     constexpr int CH = 16 / DS;                  // scores per chunk: DS S^T MFMAs (= 2 DT P V MFMAs) per half
     auto tile = [&](int t, auto buf_c, auto edge_c) {
         constexpr int buf = decltype(buf_c)::value;

@@ -1457,8 +1457,8 @@ __global__ __launch_bounds__(64 * NW, BM == 128 && !(EK & EK_DEEP) ? 2 : 1) __at
 // 3 x 3 convolutions with tiles of 96 (4 waves, 128 pixels) or 192 (8 waves, 256 pixels) output channels, a wave 96
 // channels of 32 or 64 pixels on v_mfma_f32_16x16x32_f16, over input channels in multiples of 32. A k step is one row of
 // taps (dy) and 32 channels, 96 deep: its three taps read the same BM + 2 input rows, which come in once, not once a
-// tap as in gemm_tile's 64-deep steps: 27 KB a step for 128 x 96 instead of 28 KB for 64 deep, 53 instead of 57 for 256 x
-// 192, so three stages fit (two workgroups a CU for the 96-channel tiles) and a step's direct loads have two steps to
+// tap as in gemm_tile's 64-deep steps: 27 KB a step for 128 x 96 instead of 28 KB for 64 deep, 53 instead of 57 for
+// 256 x 192, so three stages fit (two workgroups a CU for the 96-channel tiles) and a step's direct loads have two steps to
 // land. LDS rows: the weights' 192 bytes [dx][32 channels], the input's 64; 16-byte chunks swizzled by (row >> 2) & 3
 // within each 64 bytes, so 16 rows at one chunk cover all banks. One barrier a step, between its second and third tap:
 // behind it the third tap's products read the next step's first fragments and refill this step's stage. The 96-channel
@@ -2440,8 +2440,8 @@ GemmPlan gemm_plan(const mk_gemm_args* a, uint32_t n, uint32_t cus, bool conv, b
     if (narrow_ok)
         consider(256, 64, 0.62);
     if (short_ok)
-        // fp8 weights: 0.76 (their conversion; us on the best 256-token tiles -> on these: 600 x 12288 x 3072 74 -> 58, 2048
-        // x 10240 x 1280 GEGLU 76 -> 62, 1024 x 3072 x 3072 38 -> 35; 1024 x 12288 x 3072 76 and 89)
+        // fp8 weights: 0.76 (their conversion; us on the best 256-token tiles -> on these: 600 x 12288 x 3072 74 -> 58,
+        // 2048 x 10240 x 1280 GEGLU 76 -> 62, 1024 x 3072 x 3072 38 -> 35; 1024 x 12288 x 3072 76 and 89)
         consider(128, 128, f8 ? 0.76 : 0.67);
     if (best.cost < 0) // N not a multiple of 128 with an activation or GLU: the dispatch rejects it
         consider(256, 64, 0.62);

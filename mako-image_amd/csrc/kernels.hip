@@ -515,13 +515,13 @@ __global__ __launch_bounds__(256) void gemv_kernel(const float* __restrict__ x, 
     }
 }
 
-// GEMV for R rows (1 or 2) with K = 512 * KI: each wave computes 2 outputs with all 2 * KI of its 16-byte weight loads issued
-// first; while they are in flight the workgroup (8 waves, 16 outputs) converts x' to bf16 in LDS once (each wave
+// GEMV for R rows (1 or 2) with K = 512 * KI: each wave computes 2 outputs with all 2 * KI of its 16-byte weight loads
+// issued first; while they are in flight the workgroup (8 waves, 16 outputs) converts x' to bf16 in LDS once (each wave
 // converting the whole row itself cost more VALU time than the dot products), and the dot products take the bf16 pairs
 // as they are (v_dot2_f32_bf16). HBM-bound once the launch fills the chip, which 16 outputs a workgroup do from 4096
 // outputs on; 4 outputs a wave measured slower at every size (1 x 3072 x 3072 7.5 against 5.8 us, 1 x 368640 x 3072 324
 // against 312 us, 7.2 TB/s), one the same. Two rows on this form instead of gemv_kernel (scalar fp32 products, its loads
-// behind the row's staging): 4096 x 4096 42 -> 9.4 us, 16384 x 4096 70 -> 31 us.
+// behind the rows' staging): 4096 x 4096 42 -> 9.4 us, 16384 x 4096 70 -> 31 us.
 template <int KI, int R>
 __global__ __launch_bounds__(512) void gemv_rows_kernel(const float* __restrict__ x, const uint16_t* __restrict__ w,
                                                         const float* __restrict__ bias, uint32_t N,
@@ -966,8 +966,8 @@ static mk_status group_norm_run(const float* x, uint32_t batch, uint32_t rows, u
     double2* part = reinterpret_cast<double2*>(ws);
     float2* stats = reinterpret_cast<float2*>(ws + group_norm_part_bytes(batch, rows, groups));
     const uint32_t cg = c / groups, gp = std::min(groups, std::max(1u, 256u / cg));
-    group_partial_kernel<<<dim3(chunks, batch, cdiv(groups, gp)), 256, sizeof(double2) * gp * cg, s>>>(x, rows, c, groups,
-                                                                                                     gp, part);
+    const dim3 grid(chunks, batch, cdiv(groups, gp));
+    group_partial_kernel<<<grid, 256, sizeof(double2) * gp * cg, s>>>(x, rows, c, groups, gp, part);
     group_final_kernel<<<dim3(groups, batch), 64, 0, s>>>(part, chunks, groups, double(rows) * double(c / groups), eps,
                                                           stats);
     const bool vec = c % 4 == 0 && uint64_t(rows) * c < (uint64_t(1) << 32) &&
