@@ -333,6 +333,40 @@ def test_gemm_split_k(gpu, rng, Mr, N, K, epi, wdt):
     assert np.abs(outs[0] - want).max() <= tol * max(np.abs(want).max(), np.abs(y).max())
 
 
+@pytest.mark.parametrize("wdt", [M.BF16, M.FP8])
+def test_gemm_split_k_strides_and_batches(gpu, rng, wdt):
+    # two problems of two batch items each, padded rows of A and C, gaps between the items, a gate row that changes
+    # inside each item: the rows' values, and nothing outside them
+    N, K, B, split = 256, 2048, 2, 11
+    lda, ldc = K + 64, N + 8
+    if wdt == M.FP8:
+        codes = rng.integers(0, 120, (N, K)).astype(np.uint8)
+        scale = rng.uniform(0.5, 1.5, N).astype(np.float32) * 1e-3
+        Wq, Wd, sd = R.e4m3_table()[codes] * scale[:, None], dev(codes), dev(scale)
+    else:
+        Wq = R.bf16_round(rng.standard_normal((N, K)).astype(np.float32) * 0.03)
+        Wd, sd = bdev(Wq), None
+    gates, b = rng.standard_normal((2, N)).astype(np.float32), rng.standard_normal(N).astype(np.float32)
+    gd, bd = dev(gates), dev(b)
+    probs = []
+    for Mr in (150, 29):
+        A = R.bf16_round(rng.standard_normal((B, Mr + 3, lda)).astype(np.float32))
+        X = rng.standard_normal((B, Mr + 2, ldc)).astype(np.float32)
+        probs.append((Mr, A, X, bdev(A), dev(X)))
+    arr = (M.GemmArgs * 2)(*[gemm_args(Ad, Wd, bias=bd, wscale=sd, c=xd, epi=M.EPI_GATE_ADD, M_=(Mr, N, K), batch=B,
+                                       lda=lda, ldc=ldc, sa=(Mr + 3) * lda, sc=(Mr + 2) * ldc, gate=gd, gate_alt=N,
+                                       split=split, seg=Mr, w_dtype=wdt) for Mr, _, _, Ad, xd in probs])
+    M.call("mk_gemm_grouped", C.cast(arr, C.c_void_p), 2, None)
+    M.sync()
+    for Mr, A, X, _, xd in probs:
+        got = fetch(xd, X.shape)
+        y = A[:, :Mr, :K].astype(np.float64) @ Wq.T.astype(np.float64) + b
+        want = X.astype(np.float64)
+        want[:, :Mr, :N] += np.where(np.arange(Mr)[:, None] < split, gates[1], gates[0]) * y
+        assert maxrel(got[:, :Mr, :N], want[:, :Mr, :N]) < 1e-5  # fp32 sums
+        assert np.array_equal(got[:, Mr:], X[:, Mr:]) and np.array_equal(got[:, :, N:], X[:, :, N:])
+
+
 def test_gemm_split_k_grouped_on_many_streams(gpu, rng):
     # two problems a launch on more streams than there are slab buffers, all in flight together: every launch has the
     # bits of the same one run alone
