@@ -1,12 +1,37 @@
 // C ABI plumbing: error state, device / memory / stream / event calls, and the RNG key.
 #include "common.hpp"
 
+#include <algorithm>
 #include <cstdio>
+#include <mutex>
+#include <vector>
 
 namespace mk {
 
 namespace {
 thread_local std::string g_error;
+std::mutex g_streams_mutex;
+std::vector<const void*> g_streams; // the library's streams alive
+}
+
+void adopt_stream(const void* stream)
+{
+    std::lock_guard<std::mutex> lock(g_streams_mutex);
+    g_streams.push_back(stream);
+}
+
+bool known_stream(const void* stream)
+{
+    if (!stream)
+        return true;
+    std::lock_guard<std::mutex> lock(g_streams_mutex);
+    return std::find(g_streams.begin(), g_streams.end(), stream) != g_streams.end();
+}
+
+void forget_stream(const void* stream)
+{
+    std::lock_guard<std::mutex> lock(g_streams_mutex);
+    g_streams.erase(std::remove(g_streams.begin(), g_streams.end(), stream), g_streams.end());
 }
 
 void set_error(const std::string& msg) { g_error = msg; }
@@ -128,6 +153,7 @@ mk_status mk_stream_create(void** s)
         return fail(MK_ERR_ARG, "stream_create: null");
     hipStream_t st;
     MK_HIP(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
+    adopt_stream(st);
     *s = st;
     return MK_OK;
 }

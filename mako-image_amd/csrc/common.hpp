@@ -67,6 +67,12 @@ double gemm_cost(const mk_gemm_args* a, uint32_t n, uint32_t cus);
 // MK_ERR_DEVICE when a stream-K launch on `stream` (all: on any stream of any device) gave up waiting for a partial
 // tile since the last check (the check clears it); called after synchronisations of that stream (all: of the device).
 mk_status gemm_take_error(const void* stream, bool all = false);
+// Streams whose handle names one stream for as long as a workspace may remember it: the null stream and those the
+// library made, which end by release_stream (adopt_stream after their creation). A caller's handle can name several:
+// hipStreamPerThread is another stream in each thread, and a destroyed stream's handle can come back for a new one.
+void adopt_stream(const void* stream);
+bool known_stream(const void* stream);
+void forget_stream(const void* stream);
 // To be called before a stream is destroyed: waits for its last stream-K, split-K and group norm launches and frees their
 // workspaces for other streams (an event must not be asked after the stream it was recorded on is gone).
 void release_stream(const void* stream);

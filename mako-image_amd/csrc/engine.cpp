@@ -1003,6 +1003,7 @@ mk_status mk_engine_create(const mk_config* cfg, mk_engine** out)
     if (!e->cfg.max_batch)
         e->cfg.max_batch = 2;
     MK_HIP(hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking));
+    adopt_stream(e->stream);
     MK_HIP(hipStreamCreateWithFlags(&e->side, hipStreamNonBlocking));
     MK_HIP(hipEventCreateWithFlags(&e->temb_ready, hipEventDisableTiming));
     e->mod_ready.resize(e->cfg.blocks);

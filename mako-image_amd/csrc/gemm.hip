@@ -1818,8 +1818,9 @@ __global__ __launch_bounds__(64 * NW, 1) __attribute__((amdgpu_waves_per_eu(NW /
 
 // Stream-K workspaces: two partial slots and flags per workgroup of a one-a-CU grid, and the launch epoch the flags
 // are compared with (so they never need clearing). A workspace serves one launch at a time: a launch takes the
-// workspace its stream used last (stream order keeps the two apart), else one whose last launch has completed (its
-// event), else a new one, and past kSkPool workspaces a device's least recently used one after its last launch (the
+// workspace its stream used last (stream order keeps the two apart; where the handle alone does not say that it is the
+// same stream, known_stream, the launch also waits for the last one's event), else one whose last launch has completed
+// (its event), else a new one, and past kSkPool workspaces a device's least recently used one after its last launch (the
 // stream waits for that launch's event). Streams of one device thus never share partials in flight.
 // The memory is uncached: a partial written by a CU of one XCD is read by a CU of another, whose L2 is not coherent
 // with the writer's for ordinary allocations. Allocated at the full size and never freed (uncached memory a kernel has
@@ -1833,6 +1834,7 @@ struct SkWork {
     uint32_t* flags = nullptr;
     uint32_t nflags = 0, epoch = 0;
     hipStream_t last = nullptr;
+    bool known = false; // `last` was a known_stream
     hipEvent_t done = nullptr;
     bool idle = false; // its last launch's stream is gone, the launch complete: `done` names a dead stream, not asked
     uint64_t used = 0; // launch counter at its last use (least recently used first)
@@ -1864,6 +1866,26 @@ bool sk_done(const SkWork& w)
     return e == hipSuccess;
 }
 
+bool capturing(hipStream_t s)
+{
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return cap != hipStreamCaptureStatusNone;
+}
+
+// Stream s after event `done`, which may have been recorded on a stream that is gone: then after the whole device.
+mk_status wait_done(hipStream_t s, hipEvent_t done)
+{
+    if (hipStreamWaitEvent(s, done, 0) != hipSuccess) {
+        (void)hipGetLastError();
+        MK_HIP(hipDeviceSynchronize());
+    }
+    return MK_OK;
+}
+
 // A workspace for one stream-K launch of `need` partial bytes on stream s (g_sk_mutex held).
 mk_status sk_acquire(SkDevice& D, hipStream_t s, size_t need, uint32_t nflags, SkWork*& out)
 {
@@ -1871,6 +1893,8 @@ mk_status sk_acquire(SkDevice& D, hipStream_t s, size_t need, uint32_t nflags, S
     for (auto& w : D.pool)
         if (w->last == s && w->ws_bytes >= need && w->nflags >= nflags)
             pick = w.get();
+    if (pick && !pick->known && !capturing(s)) // (a capture cannot wait for an event of before it)
+        MK_TRY(wait_done(s, pick->done));
     if (!pick)
         for (auto& w : D.pool)
             if (w->ws_bytes >= need && w->nflags >= nflags && sk_done(*w)) {
@@ -1896,10 +1920,7 @@ mk_status sk_acquire(SkDevice& D, hipStream_t s, size_t need, uint32_t nflags, S
                 pick = w.get();
         if (!pick)
             return fail(MK_ERR_UNSUPPORTED, "gemm: stream-K workspaces smaller than this launch needs");
-        if (hipStreamWaitEvent(s, pick->done, 0) != hipSuccess) { // its stream is gone: wait for the whole device
-            (void)hipGetLastError();
-            MK_HIP(hipDeviceSynchronize());
-        }
+        MK_TRY(wait_done(s, pick->done));
     }
     out = pick;
     return MK_OK;
@@ -1932,14 +1953,17 @@ mk_status sk_check(SkDevice& D, hipStream_t s, bool all)
 }
 
 // Slabs of split-K launches: up to kSplitPool buffers of kSplitBytes a device, one a stream, so a stream's launches
-// follow each other on its own buffer and streams never share one. A stream beyond the pool takes the least recently
-// used buffer over after a device-wide wait; a destroyed stream's is given back by release_stream. (32 MB of slabs
-// stay in the memory-side cache between the two kernels.) Locked with g_sk_mutex over both launches.
+// follow each other on its own buffer and streams never share one. Where the handle alone does not say that it is the
+// same stream (known_stream), a launch records an event and the next one on that handle waits for it (2.8 us a launch;
+// the FFN over 77 rows, two of them, 52.5 -> 58.1 us). A stream beyond the pool takes the least recently used buffer over
+// after a device-wide wait; a destroyed stream's is given back by release_stream. (32 MB of slabs stay in the
+// memory-side cache between the two kernels.) Locked with g_sk_mutex over both launches.
 constexpr size_t kSplitBytes = size_t(32) << 20, kSplitPool = 8;
 struct SplitWork {
     float* ws = nullptr;
     hipStream_t owner = nullptr;
-    bool owned = false;
+    bool owned = false, known = false; // known: the owner is a known_stream; else `done` is behind its last launch
+    hipEvent_t done = nullptr;
     uint64_t used = 0;
 };
 struct SplitDevice {
@@ -1949,23 +1973,32 @@ struct SplitDevice {
 SplitDevice g_split[kMaxDevices];
 
 // The buffer of stream s (g_sk_mutex held); null when it cannot be had now (another stream is being captured).
-float* split_acquire(SplitDevice& D, hipStream_t s)
+SplitWork* split_acquire(SplitDevice& D, hipStream_t s)
 {
     SplitWork* pick = nullptr;
     for (auto& w : D.pool)
         if (w.owned && w.owner == s)
             pick = &w;
+    if (pick && !pick->known && wait_done(s, pick->done) != MK_OK) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
     if (!pick)
         for (auto& w : D.pool)
             if (!w.owned)
                 pick = &w;
     if (!pick && D.pool.size() < kSplitPool) {
-        void* p = nullptr;
-        if (hipMalloc(&p, kSplitBytes) != hipSuccess) {
+        SplitWork w;
+        if (hipMalloc(reinterpret_cast<void**>(&w.ws), kSplitBytes) != hipSuccess) {
             (void)hipGetLastError();
             return nullptr;
         }
-        D.pool.push_back(SplitWork{static_cast<float*>(p)});
+        if (hipEventCreateWithFlags(&w.done, hipEventDisableTiming) != hipSuccess) {
+            (void)hipGetLastError();
+            (void)hipFree(w.ws);
+            return nullptr;
+        }
+        D.pool.push_back(w);
         pick = &D.pool.back();
     }
     if (!pick) {
@@ -1979,8 +2012,9 @@ float* split_acquire(SplitDevice& D, hipStream_t s)
     }
     pick->owner = s;
     pick->owned = true;
+    pick->known = known_stream(s);
     pick->used = ++D.launches;
-    return pick->ws;
+    return pick;
 }
 
 template <int EK> void launch_reduce(const GemmG& G, const float* ws, uint32_t splits, uint64_t slab, uint32_t rows,
@@ -1997,12 +2031,7 @@ mk_status launch_split(GemmP* p, uint32_t count, const GemmPlan& plan, int ek, b
                        hipStream_t s, bool& done)
 {
     done = false;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
-        (void)hipGetLastError();
-        return MK_OK;
-    }
-    if (cap != hipStreamCaptureStatusNone)
+    if (capturing(s))
         return MK_OK;
     int dev = 0;
     MK_HIP(hipGetDevice(&dev));
@@ -2022,9 +2051,10 @@ mk_status launch_split(GemmP* p, uint32_t count, const GemmPlan& plan, int ek, b
     if (slab * splits * 4 > kSplitBytes)
         return MK_OK;
     std::lock_guard<std::mutex> lock(g_sk_mutex);
-    float* ws = split_acquire(g_split[dev], s);
-    if (!ws)
+    SplitWork* W = split_acquire(g_split[dev], s);
+    if (!W)
         return MK_OK;
+    float* const ws = W->ws;
     uint32_t r0 = 0;
     for (uint32_t i = 0; i < count; ++i) {
         GemmP& q = P.g[i];
@@ -2060,6 +2090,8 @@ mk_status launch_split(GemmP* p, uint32_t count, const GemmPlan& plan, int ek, b
     else
         launch_reduce<EK_RMW>(G, ws, splits, slab, rows, s);
     MK_HIP(hipGetLastError());
+    if (!W->known)
+        MK_HIP(hipEventRecord(W->done, s));
     done = true;
     return MK_OK;
 }
@@ -2111,6 +2143,7 @@ mk_status launch(GemmP* p, uint32_t count, const GemmPlan& plan, hipStream_t s)
             MK_HIP(hipGetLastError());
             MK_HIP(hipEventRecord(W->done, s));
             W->last = s;
+            W->known = known_stream(s);
             W->idle = false;
             W->used = ++D.launches;
             return MK_OK;
@@ -2355,6 +2388,7 @@ void release_stream(const void* stream)
                 (void)hipStreamSynchronize(w.owner);
                 w.owned = false;
             }
+    forget_stream(stream);
 }
 
 mk_status gemm_take_error(const void* stream, bool all)

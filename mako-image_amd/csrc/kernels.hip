@@ -984,17 +984,18 @@ static mk_status group_norm_run(const float* x, uint32_t batch, uint32_t rows, u
 }
 
 // mk_group_norm's partial sums: one buffer a device, grown (stream-ordered) when a call needs more and kept, so a
-// steady-state call allocates nothing. A call's stream first waits for the event of the buffer's previous user when that
-// was another stream, and records it after its own kernels: calls on different streams take turns on the buffer. A
-// stream that is about to be destroyed gives the buffer back (group_norm_release_stream): the event of a destroyed
-// stream must not be waited for.
+// steady-state call allocates nothing. A call's stream first waits for the event of the buffer's previous user unless
+// that was the same stream (the same handle, of a known_stream), and records it after its own kernels: calls on
+// different streams take turns on the buffer. A stream that is about to be destroyed gives the buffer back
+// (group_norm_release_stream): the event of a destroyed stream must not be waited for.
 struct GnScratch {
     int dev = -1;
     char* p = nullptr;
     size_t bytes = 0;
     hipEvent_t last = nullptr;
     hipStream_t owner = nullptr;
-    bool busy = false; // `owner` may still run the buffer's last user
+    bool known = false; // `owner` was a known_stream
+    bool busy = false;  // `owner` may still run the buffer's last user
 };
 static std::mutex g_gn_mutex;
 static std::vector<GnScratch> g_gn;
@@ -1029,7 +1030,7 @@ mk_status group_norm_to(const float* x, uint32_t batch, uint32_t rows, uint32_t 
         w->dev = dev;
         MK_HIP(hipEventCreateWithFlags(&w->last, hipEventDisableTiming));
     }
-    if (w->busy && w->owner != s && hipStreamWaitEvent(s, w->last, 0) != hipSuccess) {
+    if (w->busy && !(w->owner == s && w->known) && hipStreamWaitEvent(s, w->last, 0) != hipSuccess) {
         (void)hipGetLastError(); // its stream was destroyed elsewhere: wait for the whole device
         MK_HIP(hipDeviceSynchronize());
     }
@@ -1046,6 +1047,7 @@ mk_status group_norm_to(const float* x, uint32_t batch, uint32_t rows, uint32_t 
     const mk_status st = group_norm_run(x, batch, rows, c, groups, g, b, eps, y, w->p, s, y_dtype == MK_F16);
     MK_HIP(hipEventRecord(w->last, s));
     w->owner = s;
+    w->known = known_stream(s);
     w->busy = true;
     return st;
 }

@@ -696,6 +696,7 @@ struct mk_vae {
     {
         const uint32_t b = base, d0 = 4 * b;
         MK_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
+        adopt_stream(stream);
         MK_TRY(alloc(size_t(z) * z * 4, reinterpret_cast<void**>(&pq_w)));
         MK_TRY(alloc(size_t(z) * 4, reinterpret_cast<void**>(&pq_b)));
         slots["post_quant_conv.weight"] = Slot{Slot::PQ_W, nullptr, pq_w, z * z, {z, z, 1, 1}};

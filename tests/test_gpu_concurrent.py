@@ -1,6 +1,9 @@
 """Engines on separate streams at the same time: two dual-stream engines (each step's FFN-down runs as a stream-K
 launch, each stream with its own partials workspace) and an SDXL engine run concurrently, and every result equals,
 bit for bit, the same engine's result when it ran alone."""
+import ctypes as C
+import threading
+
 import numpy as np
 import pytest
 
@@ -63,3 +66,96 @@ def test_dual_and_sdxl_engines_on_separate_streams_match_their_solo_bits(gpu):
     for e, _ in duals:
         e.close()
     sx.close()
+
+
+N, K, SHAPES, GN = 256, 4096, (200, 40), (2, 1024, 640, 32)  # a grouped launch that splits its k steps; a group norm
+PER_THREAD = 2  # hipStreamPerThread: one handle, a stream of its own in each thread
+
+
+class Small:
+    """One seed's split-K GEMM and group norm on a stream, into new buffers each launch."""
+
+    def __init__(self, seed):
+        r = np.random.default_rng(seed)
+        dev = lambda a: M.Dev.from_array(a.astype(np.float32))  # noqa: E731
+        bdev = lambda a: M.Dev.from_array(M.bf16_bits(a.astype(np.float32)))  # noqa: E731
+        self.a = [bdev(r.standard_normal((m, K))) for m in SHAPES]
+        self.w, self.b = bdev(r.standard_normal((N, K)) * 0.03), dev(r.standard_normal(N))
+        self.x, self.g, self.gb = dev(r.standard_normal(GN[:3])), dev(r.standard_normal(GN[2])), dev(
+            r.standard_normal(GN[2]))
+        self.runs = []
+
+    def out(self):
+        c = [M.Dev(m * N * 4) for m in SHAPES]
+        args = []
+        for a, m, o in zip(self.a, SHAPES, c):
+            g = M.GemmArgs()
+            g.a, g.w, g.bias, g.c = a.p, self.w.p, self.b.p, o.p
+            g.M, g.N, g.K, g.lda, g.ldc, g.batch = m, N, K, K, N, 1
+            g.w_dtype, g.c_dtype, g.epilogue = M.BF16, M.F32, M.EPI_STORE
+            args.append(g)
+        return (M.GemmArgs * 2)(*args), c, M.Dev(GN[0] * GN[1] * GN[2] * 2)
+
+    def launch(self, stream, bufs):
+        arr, c, y = bufs
+        M.call("mk_gemm_grouped", C.cast(arr, C.c_void_p), 2, stream)
+        M.call("mk_group_norm", self.x.p, *GN, self.g.p, self.gb.p, 1e-6, y.p, stream)
+        self.runs.append(bufs)
+
+    def read(self):
+        got = [[d.to_array(np.float32, (m, N)) for d, m in zip(c, SHAPES)] + [y.to_array(np.uint16, GN[:3])]
+               for _, c, y in self.runs]
+        self.runs = []
+        return got
+
+
+def test_threads_on_their_per_thread_streams_match_their_solo_bits(gpu):
+    # hipStreamPerThread is the same handle in every thread: the workspaces of one thread's launches are not another's
+    work = [Small(s) for s in range(4)]
+    solo = []
+    for w in work:
+        w.launch(None, w.out())
+        M.sync()
+        solo.append(w.read()[0])
+    start, errors = threading.Barrier(len(work)), []
+
+    def run(w, bufs):
+        try:
+            start.wait()
+            for b in bufs:
+                w.launch(PER_THREAD, b)
+            M.call("mk_stream_synchronize", PER_THREAD)
+        except Exception as e:  # noqa: BLE001
+            errors.append(e)
+
+    threads = [threading.Thread(target=run, args=(w, [w.out() for _ in range(20)])) for w in work]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors
+    for w, want in zip(work, solo):
+        for i, got in enumerate(w.read()):
+            assert all(np.array_equal(a, b) for a, b in zip(got, want)), f"launch {i}"
+
+
+def test_streams_destroyed_by_their_caller_match_their_solo_bits(gpu):
+    # a stream that its caller made and destroys with work in flight, and the next one, which may get its handle
+    hip = C.CDLL("libamdhip64.so.7")
+    work = [Small(s) for s in range(2)]
+    solo = []
+    for w in work:
+        w.launch(None, w.out())
+        M.sync()
+        solo.append(w.read()[0])
+    bufs = [[w.out() for w in work] for _ in range(12)]
+    for pair in bufs:
+        for w, b in zip(work, pair):
+            s = C.c_void_p()
+            assert hip.hipStreamCreateWithFlags(C.byref(s), 1) == 0  # non-blocking
+            w.launch(s.value, b)
+            assert hip.hipStreamDestroy(s) == 0
+    M.sync()
+    for w, want in zip(work, solo):
+        for i, got in enumerate(w.read()):
+            assert all(np.array_equal(a, b) for a, b in zip(got, want)), f"launch {i}"
