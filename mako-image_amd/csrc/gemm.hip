@@ -1853,14 +1853,12 @@ std::mutex g_sk_mutex;
 SkDevice g_sk[kMaxDevices];
 uint32_t g_sk_polls = kSkPollsDefault;
 
-// Whether a workspace's last launch has completed. The event's state lies with the stream it was recorded on: a
+// Whether the work in front of an event has completed. The event's state lies with the stream it was recorded on: a
 // stream that a caller destroyed behind the library's back makes the query fail, and that error would otherwise be
-// reported by the next launch (such a workspace counts as busy).
-bool sk_done(const SkWork& w)
+// reported by the next launch (such an event counts as not reached).
+bool event_done(hipEvent_t done)
 {
-    if (w.idle)
-        return true;
-    const hipError_t e = hipEventQuery(w.done);
+    const hipError_t e = hipEventQuery(done);
     if (e != hipSuccess && e != hipErrorNotReady)
         (void)hipGetLastError();
     return e == hipSuccess;
@@ -1897,7 +1895,7 @@ mk_status sk_acquire(SkDevice& D, hipStream_t s, size_t need, uint32_t nflags, S
         MK_TRY(wait_done(s, pick->done));
     if (!pick)
         for (auto& w : D.pool)
-            if (w->ws_bytes >= need && w->nflags >= nflags && sk_done(*w)) {
+            if (w->ws_bytes >= need && w->nflags >= nflags && (w->idle || event_done(w->done))) {
                 pick = w.get();
                 break;
             }
@@ -1955,38 +1953,53 @@ mk_status sk_check(SkDevice& D, hipStream_t s, bool all)
 // Slabs of split-K launches: up to kSplitPool buffers of kSplitBytes a device, one a stream, so a stream's launches
 // follow each other on its own buffer and streams never share one. Where the handle alone does not say that it is the
 // same stream (known_stream), a launch records an event and the next one on that handle waits for it (2.8 us a launch;
-// the FFN over 77 rows, two of them, 52.5 -> 58.1 us). A stream beyond the pool takes the least recently used buffer over
-// after a device-wide wait; a destroyed stream's is given back by release_stream. (32 MB of slabs stay in the
-// memory-side cache between the two kernels.) Locked with g_sk_mutex over both launches.
+// the FFN over 77 rows, two of them, 52.5 -> 58.1 us). A stream without a buffer takes a free one, one whose event is
+// reached, a new one, or the least recently used one behind its event: the stream waits for that, not the host. Once
+// more streams than buffers have come by, every launch records its event. A destroyed stream's buffer is given back by
+// release_stream. (32 MB of slabs stay in the memory-side cache between the two kernels.) Locked with g_sk_mutex over
+// both launches.
 constexpr size_t kSplitBytes = size_t(32) << 20, kSplitPool = 8;
 struct SplitWork {
     float* ws = nullptr;
     hipStream_t owner = nullptr;
-    bool owned = false, known = false; // known: the owner is a known_stream; else `done` is behind its last launch
+    bool owned = false, known = false; // known: the owner is a known_stream
     hipEvent_t done = nullptr;
+    bool marked = false; // `done` is behind its last launch
     uint64_t used = 0;
 };
 struct SplitDevice {
     uint64_t launches = 0;
+    bool crowded = false; // a stream has found every buffer owned
     std::vector<SplitWork> pool;
 };
 SplitDevice g_split[kMaxDevices];
 
-// The buffer of stream s (g_sk_mutex held); null when it cannot be had now (another stream is being captured).
+// Stream s after the last launch on buffer w: false where that cannot be waited for now (it left no event, and its
+// stream is being captured).
+bool split_take(SplitWork& w, hipStream_t s)
+{
+    if (!w.marked && (capturing(w.owner) || hipEventRecord(w.done, w.owner) != hipSuccess)) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return wait_done(s, w.done) == MK_OK;
+}
+
+// The buffer of stream s (g_sk_mutex held); null when it cannot be had now.
 SplitWork* split_acquire(SplitDevice& D, hipStream_t s)
 {
     SplitWork* pick = nullptr;
     for (auto& w : D.pool)
         if (w.owned && w.owner == s)
             pick = &w;
-    if (pick && !pick->known && wait_done(s, pick->done) != MK_OK) {
-        (void)hipGetLastError();
+    if (pick && !pick->known && wait_done(s, pick->done) != MK_OK)
         return nullptr;
-    }
     if (!pick)
         for (auto& w : D.pool)
-            if (!w.owned)
+            if (!w.owned || (w.marked && event_done(w.done))) {
                 pick = &w;
+                break;
+            }
     if (!pick && D.pool.size() < kSplitPool) {
         SplitWork w;
         if (hipMalloc(reinterpret_cast<void**>(&w.ws), kSplitBytes) != hipSuccess) {
@@ -2002,13 +2015,12 @@ SplitWork* split_acquire(SplitDevice& D, hipStream_t s)
         pick = &D.pool.back();
     }
     if (!pick) {
-        if (hipDeviceSynchronize() != hipSuccess) {
-            (void)hipGetLastError();
-            return nullptr;
-        }
+        D.crowded = true;
         for (auto& w : D.pool)
             if (!pick || w.used < pick->used)
                 pick = &w;
+        if (!split_take(*pick, s))
+            return nullptr;
     }
     pick->owner = s;
     pick->owned = true;
@@ -2090,7 +2102,8 @@ mk_status launch_split(GemmP* p, uint32_t count, const GemmPlan& plan, int ek, b
     else
         launch_reduce<EK_RMW>(G, ws, splits, slab, rows, s);
     MK_HIP(hipGetLastError());
-    if (!W->known)
+    W->marked = !W->known || g_split[dev].crowded;
+    if (W->marked)
         MK_HIP(hipEventRecord(W->done, s));
     done = true;
     return MK_OK;
@@ -2386,7 +2399,7 @@ void release_stream(const void* stream)
         for (auto& w : D.pool)
             if (w.owned && w.owner == stream) {
                 (void)hipStreamSynchronize(w.owner);
-                w.owned = false;
+                w.owned = w.marked = false;
             }
     forget_stream(stream);
 }

@@ -3,6 +3,7 @@ launch, each stream with its own partials workspace) and an SDXL engine run conc
 bit for bit, the same engine's result when it ran alone."""
 import ctypes as C
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -159,3 +160,44 @@ def test_streams_destroyed_by_their_caller_match_their_solo_bits(gpu):
     for w, want in zip(work, solo):
         for i, got in enumerate(w.read()):
             assert all(np.array_equal(a, b) for a, b in zip(got, want)), f"launch {i}"
+
+
+def test_split_launches_on_more_streams_than_slab_buffers_do_not_wait_for_the_device(gpu):
+    # 11 streams take turns with 8 buffers while another one works: the launches return, and have their solo bits
+    work = Small(0)
+    work.launch(None, work.out())
+    M.sync()
+    want = work.read()[0]
+    streams = []
+    for _ in range(11):
+        h = C.c_void_p()
+        M.call("mk_stream_create", C.byref(h))
+        streams.append(h.value)
+    rows = 8192
+    a, w, c = M.Dev(rows * K * 2), M.Dev(rows * K * 2), M.Dev(rows * rows * 4)
+    for d in (a, w):
+        M.call("mk_memset", d.p, 0, d.nbytes)
+    g = M.GemmArgs()
+    g.a, g.w, g.c = a.p, w.p, c.p
+    g.M, g.N, g.K, g.lda, g.ldc, g.batch = rows, rows, K, K, rows, 1
+    g.w_dtype, g.c_dtype, g.epilogue = M.BF16, M.F32, M.EPI_STORE
+    for s in streams:  # every stream has had a buffer
+        work.launch(s, work.out())
+    bufs = [work.out() for _ in range(3) for _ in streams]
+    M.sync()
+    for _ in range(300):  # 0.1 s or more
+        M.call("mk_gemm", C.byref(g), streams[0])
+    t0 = time.perf_counter()
+    for b, s in zip(bufs, 3 * streams):
+        M.call("mk_gemm_grouped", C.cast(b[0], C.c_void_p), 2, s)
+    t1 = time.perf_counter()
+    M.sync()
+    t2 = time.perf_counter()
+    assert t1 - t0 < (t2 - t0) / 2, f"{(t1 - t0) * 1e3:.1f} ms of {(t2 - t0) * 1e3:.1f} for the launches"
+    for _, c, _ in bufs:
+        for d, m, x in zip(c, SHAPES, want):
+            assert np.array_equal(d.to_array(np.float32, (m, N)), x)
+    for got in work.read():
+        assert all(np.array_equal(x, y) for x, y in zip(got, want))
+    for s in streams:
+        M.call("mk_stream_destroy", s)
