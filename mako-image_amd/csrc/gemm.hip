@@ -1874,6 +1874,14 @@ bool capturing(hipStream_t s)
     return cap != hipStreamCaptureStatusNone;
 }
 
+// Lets this thread allocate and ask events while another stream is being captured (in the default mode such a call ends
+// that stream's capture; none of them concerns it).
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 // Stream s after event `done`, which may have been recorded on a stream that is gone: then after the whole device.
 mk_status wait_done(hipStream_t s, hipEvent_t done)
 {
@@ -1992,7 +2000,12 @@ SplitWork* split_acquire(SplitDevice& D, hipStream_t s)
     for (auto& w : D.pool)
         if (w.owned && w.owner == s)
             pick = &w;
-    if (pick && !pick->known && wait_done(s, pick->done) != MK_OK)
+    if (pick && pick->known) {
+        pick->used = ++D.launches;
+        return pick;
+    }
+    const RelaxedCapture relaxed;
+    if (pick && wait_done(s, pick->done) != MK_OK)
         return nullptr;
     if (!pick)
         for (auto& w : D.pool)

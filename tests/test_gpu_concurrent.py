@@ -201,3 +201,47 @@ def test_split_launches_on_more_streams_than_slab_buffers_do_not_wait_for_the_de
         assert all(np.array_equal(x, y) for x, y in zip(got, want))
     for s in streams:
         M.call("mk_stream_destroy", s)
+
+
+def test_small_gemms_during_another_streams_capture(gpu):
+    # one stream is being captured while others run split launches for the first time (they need slab buffers); the
+    # captured launches, of sizes that split when they are not captured, run whole tiles, the same bits every replay
+    hip = C.CDLL("libamdhip64.so.7")
+    work = Small(0)
+    work.launch(None, work.out())
+    M.sync()
+    want = work.read()[0]
+    handles = [C.c_void_p() for _ in range(11)]
+    for h in handles:
+        M.call("mk_stream_create", C.byref(h))
+    cap, *others = [h.value for h in handles]
+    inside, outside = work.out(), [work.out() for _ in others]
+    graph, run = C.c_void_p(), C.c_void_p()
+    assert hip.hipStreamBeginCapture(C.c_void_p(cap), 0) == 0  # global mode
+    M.call("mk_gemm_grouped", C.cast(inside[0], C.c_void_p), 2, cap)
+    for s, b in zip(others, outside):
+        M.call("mk_gemm_grouped", C.cast(b[0], C.c_void_p), 2, s)
+    assert hip.hipStreamEndCapture(C.c_void_p(cap), C.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(C.byref(run), graph, None, None, 0) == 0
+    M.sync()
+    for _, c, _ in outside:
+        assert all(np.array_equal(d.to_array(np.float32, (m, N)), x) for d, m, x in zip(c, SHAPES, want))
+    first = None
+    for _ in range(3):
+        for d in inside[1]:
+            M.call("mk_memset", d.p, 0xFF, d.nbytes)
+        M.sync()
+        assert hip.hipGraphLaunch(run, C.c_void_p(cap)) == 0
+        M.call("mk_stream_synchronize", cap)
+        got = [d.to_array(np.float32, (m, N)) for d, m in zip(inside[1], SHAPES)]
+        first = first or got
+        for g, f, x in zip(got, first, want):
+            assert np.array_equal(g, f)
+            # fp32 sums of K products in another order
+            assert np.abs(g - x).max() <= 1e-5 * np.abs(x).max()
+        work.launch(None, outside[0])  # the program's own work between the replays
+        M.sync()
+        assert all(np.array_equal(a, b) for a, b in zip(work.read()[0], want))
+    assert hip.hipGraphExecDestroy(run) == 0 and hip.hipGraphDestroy(graph) == 0
+    for s in (cap, *others):
+        M.call("mk_stream_destroy", s)
