@@ -90,13 +90,13 @@ template <> struct Elem<true> {
 };
 
 // The running max enters the S^T MFMAs as one more 16-deep product, a constant fragment of ones (K side, dim 0) times a
-// fragment holding -m (Q side), so S - m comes out of the matrix core, and the row sums are taken on the 16-bit
-// probabilities the P V product uses (v_dot2 against ones), which halves those adds too. m is kept representable in the
-// type so the product subtracts it exactly.
+// fragment holding -m (Q side), so S - m comes out of the matrix core, and the unit scale's row sums are taken on the
+// 16-bit probabilities the P V product uses (v_dot2 against ones), which halves those adds too. m is kept representable in
+// the type so the product subtracts it exactly.
 // U: K carries the softmax scale in log2 units (scale 0 at the API), so the softmax needs no per-score multiply at all;
 // a general scale multiplies each S - m by c. (The general scale had a tile of its own, a max, a multiply-add and an
-// add a score between the MFMAs instead of in their shadow: 493 -> 463 us for 2 x 24 heads of 128 over 4352 rows, 1006
-// TFLOP/s.)
+// add a score between the MFMAs instead of in their shadow: 493 -> 463 us for 2 x 24 heads of 128 over 4352 rows; on
+// another box 427 us with its row sums by v_dot2 on the 16-bit probabilities, 420 with them in fp32, 1.11 PFLOP/s.)
 // NW waves a workgroup (32 queries each): 4, or 2 for launches of few query blocks (64-dim heads), whose 64-query
 // workgroups then spread over every CU, four a CU.
 template <int D, bool U, bool F16, bool HOLE, int NW = 4>
@@ -184,14 +184,15 @@ __global__ __launch_bounds__(64 * NW, 2) __attribute__((amdgpu_waves_per_eu(2, 2
     };
     // S^T of a 32-key half of a tile: value r <-> key 8(r/4) + 4hk + r%4 of the half
     // ones at dim 0 (K side); -m at dim 0 (Q side), lanes of the first k half. A general scale's scores are unscaled
-    // products, which can pass the half range: m is then the sum of two bf16 values (dims 0 and 2; 16 bits, so that a
-    // score of 10^5 in log2 units is still met to half a unit), and this one product bf16
+    // products, which can pass the half range, and any size: m is then an fp32 value, the sum of three bf16 ones (dims 0,
+    // 2 and 3), and this one product bf16. (Two of them leave 2^-17 of m: at scores of 10^6 in log2 units that is 8, and
+    // half probabilities underflow.)
     typedef Elem<F16 && U> XM;
     typedef typename XM::v8 MV8;
     typedef typename XM::e ME;
     MV8 kone = {}, qm = {};
     if (hk == 0)
-        kone[0] = kone[2] = (ME)1.0f;
+        kone[0] = kone[2] = kone[3] = (ME)1.0f;
     // a masked key range: the same product also adds bias(key) x 1 at dim 1, bias -inf for the masked keys
     // (0 otherwise), so their scores leave the matrix core as -inf (lanes of the first k half hold dims 0 .. 7)
     if (HOLE && hk == 0)
@@ -210,6 +211,16 @@ __global__ __launch_bounds__(64 * NW, 2) __attribute__((amdgpu_waves_per_eu(2, 2
     // 2^(c x): the unit scale's scores are in log2 units already
     const float c = p.c;
     auto exp_c = [&](float x) { return __builtin_amdgcn_exp2f(U ? x : x * c); };
+    // two probabilities for the P V product, added to the row sum ls: at the unit scale as that product takes them (16
+    // bits, one v_dot2), at a general scale in fp32
+    auto prob2 = [&](float x0, float x1, uint32_t& pw, float& ls) {
+        const float e0 = exp_c(x0), e1 = exp_c(x1);
+        pw = X::pack(e0, e1);
+        if constexpr (U)
+            ls = X::sum2(pw, ls);
+        else
+            ls += e0 + e1;
+    };
     const int qpos = int(p.q_pos0) + q0 + r32;
     const bool wave_causal = uint32_t(int(p.q_pos0) + q0) < p.block;
     issue(0, 0);
@@ -260,8 +271,7 @@ __global__ __launch_bounds__(64 * NW, 2) __attribute__((amdgpu_waves_per_eu(2, 2
                     sc[2 * j] = x0;
                     sc[2 * j + 1] = x1;
                 }
-                pw[j] = X::pack(exp_c(x0), exp_c(x1));
-                ls = X::sum2(pw[j], ls);
+                prob2(x0, x1, pw[j], ls);
                 // pinned here: the redo path overwrites them, so the compiler would otherwise sink the
                 // speculative work out of the MFMA shadow into the path that keeps it
                 asm volatile("" : "+v"(pw[j]), "+v"(ls));
@@ -272,12 +282,12 @@ __global__ __launch_bounds__(64 * NW, 2) __attribute__((amdgpu_waves_per_eu(2, 2
         auto redo = [&](f32x16& sc, uint32_t (&pw)[8], float& lh, bool first, f32x16* other) {
             const float mx = max_xor32(max16(sc));
             const float mt = m + (first ? mx : fmaxf(mx, 0.0f)), m1 = float((ME)mt);
-            const float m2 = U ? 0.0f : float((ME)(mt - m1)), mn = m1 + m2;
-            const float dm = mn - m;
+            const float m2 = U ? 0.0f : float((ME)(mt - m1)), m3 = U ? 0.0f : float((ME)(mt - m1 - m2));
+            const float mn = U ? m1 : m1 + (m2 + m3), dm = mn - m;
             const float alpha = first ? 1.0f : exp_c(-dm);
             m = mn;
             if (hk == 0)
-                qm[0] = (ME)(-m1), qm[2] = (ME)(-m2);
+                qm[0] = (ME)(-m1), qm[2] = (ME)(-m2), qm[3] = (ME)(-m3);
             l *= alpha;
 #pragma unroll
             for (int r = 0; r < 16; ++r)
@@ -294,8 +304,7 @@ __global__ __launch_bounds__(64 * NW, 2) __attribute__((amdgpu_waves_per_eu(2, 2
             float ls = 0.0f;
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
-                pw[j] = X::pack(exp_c(sc[2 * j]), exp_c(sc[2 * j + 1]));
-                ls = X::sum2(pw[j], ls);
+                prob2(sc[2 * j], sc[2 * j + 1], pw[j], ls);
             }
             lh = ls;
         };

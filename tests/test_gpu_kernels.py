@@ -1367,10 +1367,11 @@ def test_attention_masked_key_range(gpu, rng, d, Tq, Tk, holes, scale):
 
 # The general scale's running max is a raw product: scores past the half range (inputs of +-60 at d = 128), a max that
 # jumps by more than 8 in log2 units on a middle and on the last tile, a negative scale, tiny scales, a causal prefix
-# and a cut last tile, in both types
+# and a cut last tile, in both types; whole scores of 21 bits at a scale that makes one of them e^8 (the max has to be met to
+# the last one)
 @pytest.mark.parametrize("dtype", [M.BF16, M.F16])
 @pytest.mark.parametrize("d,scale,mag,block", [(128, 128 ** -0.5, 60.0, 0), (64, 0.125, 3.0, 40), (128, -0.05, 1.0, 0),
-                                               (64, 1e-6, 1.0, 0), (64, 4.0, 1.0, 200)])
+                                               (64, 1e-6, 1.0, 0), (64, 4.0, 1.0, 200), (128, 8.0, 251.0, 0)])
 def test_attention_general_scale_range(gpu, rng, dtype, d, scale, mag, block):
     H, T = 2, 200
     q_pad, k_pad = 256, 256
@@ -1380,6 +1381,8 @@ def test_attention_general_scale_range(gpu, rng, dtype, d, scale, mag, block):
         q, k = np.sign(q) * 60.0, np.sign(k) * 60.0
         k[:, :, 70] = q[:, :, 5]    # 460 800 for query 5, far above its other scores
         k[:, :, 199] = q[:, :, 90]
+    if mag == 251.0:
+        q, k = np.sign(q) * 251.0, np.sign(k) * rng.integers(200, 256, k.shape).astype(np.float32)
     v = rnd(rng.standard_normal((1, H, T, d)).astype(np.float32))
     Q, Kd = np.zeros((H, q_pad, d), np.float32), np.zeros((H, k_pad, d), np.float32)
     Vt = np.zeros((H, d, k_pad), np.float32)
