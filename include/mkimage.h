@@ -301,6 +301,9 @@ mk_status mk_vae_decode(mk_vae* v, const float* tokens, size_t n, uint32_t h, ui
 /* the same on device buffers, queued on the VAE's stream (mk_vae_stream) */
 mk_status mk_vae_decode_device(mk_vae* v, const float* tokens, uint32_t h, uint32_t w, float* rgba);
 mk_status mk_vae_stream(mk_vae* v, void** stream);
+/* Whether a level of h x w pixels and c channels (a multiple of 192) writes the next level's grid from its last
+ * convolution's epilogue on a device of cus compute units (host only; a test hook). No counterpart in the reference. */
+mk_status mk_vae_up_plan(uint32_t h, uint32_t w, uint32_t c, uint32_t cus, uint32_t* out);
 
 /* ------------------------------------------------------------------------------------------------------------
  * Checkpoint files: safetensors (the reference's safetensors::Files, tests/safetensors_test.cpp:36-98). Host code

@@ -2699,6 +2699,62 @@ extern "C" mk_status mk_gemm_set_wait_limit(uint32_t polls)
 }
 
 namespace mk {
+// The tiles of a convolution over h x w pixels (g: its product over the padded rows): over the pixels when the plan for
+// h w rows has a tile height that divides w (then pixels = true), else over the padded rows.
+static GemmPlan conv_plan(const mk_gemm_args& g, uint32_t h, uint32_t w, uint32_t cus, bool by_row, bool norm, bool up,
+                          bool& pixels)
+{
+    mk_gemm_args gp = g;
+    gp.M = h * w;
+    GemmPlan plan = gemm_plan(&gp, 1, cus, true, by_row);
+    if (norm) { // the norm epilogues' tiles span the row: 128 x 96 or 256 x 192
+        plan.bm = g.N == 96 ? 128 : 256;
+        plan.bn = int(g.N);
+    }
+    if (up) {
+        plan.bm = 256;
+        plan.bn = 192;
+    }
+    // 96-channel tiles of 256 pixels (conv_kernel) from two rounds of them on, two a CU (one round and less of 128-pixel
+    // tiles keep more workgroups in flight: 128 x 128 pixels of 384 channels are 512 of them, 56 us)
+    const bool tall = by_row && plan.bn == 96 && uint64_t(gp.M) * (g.N / 96) >= uint64_t(256) * 4 * cus;
+    if (tall)
+        plan.bm = 256;
+    pixels = w % uint32_t(plan.bm) == 0;
+    if (!pixels && !norm && !up) {
+        plan = gemm_plan(&g, 1, cus, true, by_row);
+        if (tall && plan.bn == 96)
+            plan.bm = 256;
+    }
+    plan.sk = false;
+    return plan;
+}
+
+// Whether a convolution whose sums go to the nearest-2x grid of the next level (EK_RMWUP) writes them from its epilogue.
+// That epilogue runs on 256 x 192 tiles only and stores four pixels for one, all workgroups of a round at once; the pass
+// of its own reads the sums again. At widths that are no multiple of 256 it pays where the convolution takes these tiles
+// anyway (where it does not, other tiles fill its rounds better) and either the last of two rounds is nearly full or
+// there are more. Decodes with the epilogue against the pass, 256 compute units: 384 channels, 208 x 304 pixels (504
+// tiles) -20 us, 224 x 340 (604) -34, 310 x 372 (930) -85, but 2 rounds of 402 to 452 tiles +10 to +30 and, on tiles
+// of 96 channels otherwise, 216 x 304 (522) +20, 208 x 320 (530) +22; 192 channels, 416 x 608 (997) -70, 304 x 576 (691) -20,
+// 288 x 464 (528, 96 channels otherwise) +7.
+bool conv3x3_up_pays(uint32_t h, uint32_t w, uint32_t c, uint32_t n, uint32_t cus)
+{
+    if (w % 256 == 0)
+        return true;
+    mk_gemm_args g{};
+    g.M = (h + 2) * (w + 2);
+    g.N = n;
+    g.K = 9 * c;
+    g.batch = 1;
+    g.w_dtype = MK_F16;
+    g.epilogue = MK_EPI_ADD;
+    bool pixels = false;
+    const GemmPlan plan = conv_plan(g, h, w, cus, c % 32 == 0, false, false, pixels);
+    const uint64_t tiles = uint64_t(cdiv(g.M, 256)) * (n / 192);
+    return plan.bm == 256 && plan.bn == 192 && (tiles > 2 * uint64_t(cus) || tiles * 20 >= 2 * uint64_t(cus) * 19);
+}
+
 // 3 x 3 convolution as one GEMM over the padded pixel grid: output row r (grid pixel r of (h + 2) x (w + 2)) and tap
 // (dy, dx) read input row r + dy (w + 2) + dx of x, whose w + 3 slack rows before the grid make every shift
 // non-negative. K = 9 c runs tap-major: with c a multiple of 64 each 64-wide k step lies inside one tap, so the tap
@@ -2759,32 +2815,13 @@ mk_status conv3x3_run(const mk_conv_args* a, uint32_t lda, bool dense, const Con
     int cus = 0, dev = 0;
     MK_HIP(hipGetDevice(&dev));
     MK_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    // tiles over the pixels when the plan for h w rows has a tile height dividing w, else over the padded rows
-    mk_gemm_args gp = g;
-    gp.M = a->h * a->width;
-    GemmPlan plan = gemm_plan(&gp, 1, uint32_t(cus > 0 ? cus : 1), true, by_row);
-    if (nm) { // the norm epilogues' tiles span the row: 128 x 96 or 256 x 192
-        plan.bm = a->n == 96 ? 128 : 256;
-        plan.bn = a->n;
-    }
-    if (up) {
-        plan.bm = 256;
-        plan.bn = 192;
-    }
-    // 96-channel tiles of 256 pixels (conv_kernel) from two rounds of them on, two a CU (one round and less of 128-pixel
-    // tiles keep more workgroups in flight: 128 x 128 pixels of 384 channels are 512 of them, 56 us)
-    const bool tall = by_row && plan.bn == 96 && uint64_t(gp.M) * (a->n / 96) >= uint64_t(256) * 4 * uint64_t(cus);
-    if (tall)
-        plan.bm = 256;
-    if (a->width % plan.bm == 0) {
+    bool pixels = false;
+    const GemmPlan plan = conv_plan(g, a->h, a->width, uint32_t(cus > 0 ? cus : 1), by_row, nm != nullptr, up != nullptr,
+                                    pixels);
+    if (pixels) {
         p.conv_w = a->width;
-        p.conv_pix = gp.M;
-    } else if (!nm && !up) {
-        plan = gemm_plan(&g, 1, uint32_t(cus > 0 ? cus : 1), true, by_row);
-        if (tall && plan.bn == 96)
-            plan.bm = 256;
+        p.conv_pix = a->h * a->width;
     }
-    plan.sk = false;
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool add = a->epilogue == MK_EPI_ADD;
     constexpr int C = EK_CONV | EK_F16, Q = EK_CONV | EK_CONVQ | EK_F16;
@@ -2873,3 +2910,11 @@ mk_status conv3x3_up(const mk_conv_args* a, const ConvUp& up, void* stream)
     return conv3x3_run(a, a ? a->c : 0, false, nullptr, stream, &up);
 }
 } // namespace mk
+
+extern "C" mk_status mk_vae_up_plan(uint32_t h, uint32_t w, uint32_t c, uint32_t cus, uint32_t* out)
+{
+    if (!out || !h || !w || h > (1u << 14) || w > (1u << 14) || !c || c % 192 || c > 4096 || !cus)
+        return fail(MK_ERR_ARG, "vae_up_plan: null argument, no pixels, channels not a multiple of 192 or no compute units");
+    *out = conv3x3_up_pays(h, w, c, c, cus) ? 1 : 0;
+    return MK_OK;
+}

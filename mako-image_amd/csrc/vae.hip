@@ -1063,6 +1063,10 @@ struct mk_vae {
         MK_TRY(ensure(t, most * 4));
         MK_TRY(ensure(a, most * 2));
         MK_TRY(ensure(sc, most * 2));
+        int cus = 0, dev = 0;
+        MK_HIP(hipGetDevice(&dev));
+        MK_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+        cus = std::max(cus, 1);
         GridDims g{2 * th, 2 * tw};
         vae_in_kernel<<<blocks_for(g.rows() * conv_in.cip()), 256, 0, stream>>>(
             tokens, tw, g, z, conv_in.cip(), d_mean, d_sd, pq_w, pq_b, static_cast<uint16_t*>(a.p));
@@ -1086,13 +1090,12 @@ struct mk_vae {
         for (int i = 0; i < 4; ++i) {
             Up& u = ups[i];
             // the last res block's conv2 can write the nearest-2x grid the upsampling conv reads (into sc, since its
-            // input may be a) from 256 x 192 tiles: where those cover whole image rows, and at other widths where
-            // they are about two rounds of 256 compute units (832 x 1216: the two convolutions 171 -> 214 and 216 -> 288 us,
-            // vae_up's 76 + 173 us gone); the smaller levels keep the convolution's own tiles and vae_up
+            // input may be a), where that is faster than vae_up (832 x 1216: the two convolutions 171 -> 214 and 216 ->
+            // 288 us, vae_up's 76 + 173 us gone)
             const Res& rl = u.res[2];
             const bool up_fused = u.up && !rl.shortcut && !rl.c2.dense && rl.c2.co % 192 == 0 &&
                                   rl.c2.cop() == rl.c2.co && u.cout == rl.c2.co && u.conv.cip() == rl.c2.co &&
-                                  (g.w % 256 == 0 || g.grid_rows() / 256 * (rl.c2.co / 192) >= 500);
+                                  conv3x3_up_pays(g.h, g.w, rl.c2.ci, rl.c2.co, uint32_t(cus));
             uint16_t* const upbuf = up_fused ? ns : na;
             for (int j = 0; j < 3; ++j) {
                 const Res& r = u.res[j];

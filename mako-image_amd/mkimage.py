@@ -154,6 +154,7 @@ _SIGS = {
     "mk_vae_decode": (_i, [_vp, _vp, _sz, _u32, _u32, _vp]),
     "mk_vae_decode_device": (_i, [_vp, _vp, _u32, _u32, _vp]),
     "mk_vae_stream": (_i, [_vp, C.POINTER(_vp)]),
+    "mk_vae_up_plan": (_i, [_u32, _u32, _u32, _u32, C.POINTER(_u32)]),
     "mk_vae_set_probe": (_i, [_vp, PROBE, _vp]),
 }
 

@@ -110,3 +110,21 @@ def test_noise_matches_the_oracle_bit_for_bit():
         assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), seed
     # one draw is the first of a pair; two calls of one draw each are the same first value
     assert mkimage.noise(7, 1)[0] == mkimage.noise(7, 2)[0]
+
+
+def test_vae_up_plan():
+    # the 2x grid is written by the convolution where that measured faster than the pass of its own (256 compute units):
+    # any width of whole tiles; else convolutions on 256 x 192 tiles in more than two rounds, or two nearly full ones
+    def plan(h, w, c, cus=256):
+        out = ctypes.c_uint32(7)
+        mkimage.call("mk_vae_up_plan", h, w, c, cus, ctypes.byref(out))
+        return out.value
+
+    assert [plan(h, w, 384) for h, w in ((304, 208), (340, 224), (256, 256), (464, 260), (372, 310))] == [1] * 5
+    # other tiles, two rounds of 402 to 452 tiles, a small level
+    assert [plan(h, w, 384) for h, w in ((304, 216), (320, 208), (280, 180), (320, 176), (152, 104))] == [0] * 5
+    assert [plan(h, w, 192) for h, w in ((608, 416), (456, 272), (576, 304), (288, 512))] == [1] * 4
+    assert [plan(h, w, 192) for h, w in ((464, 288), (368, 360), (304, 240), (48, 48))] == [0] * 4
+    # rounds are the device's: twice the image on twice the units, half of it on half
+    assert plan(608, 208, 384, 512) == plan(304, 208, 384, 256) == plan(152, 208, 384, 128) == 1
+    assert mkimage.lib().mk_vae_up_plan(304, 208, 100, 256, ctypes.byref(ctypes.c_uint32())) == 1

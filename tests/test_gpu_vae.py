@@ -154,11 +154,12 @@ def test_vae_decode_matches_oracle(gpu, base, h, w):
     assert np.array_equal(vae.decode(tokens, h, w), got)
 
 
-def test_vae_decode_of_a_width_no_tile_divides(gpu):
-    # 45 x 46 tokens: the 192-channel level (360 x 368 pixels) writes the 2x grid from tiles over the padded rows, and
-    # the mid block's 8280 pixels are padded to whole 256-wide tiles; against the decoder in torch's fp32, its
-    # convolutions' operands rounded to half as the kernels' are
-    base, h, w = 96, 45, 46
+# 34 x 57 tokens: the 192-channel level (272 x 456 pixels) writes the 2x grid from tiles over the padded rows; 45 x 46 (360 x
+# 368) does not, and the mid block's 8280 pixels are padded to whole 256-wide tiles; against the decoder in torch's fp32,
+# its convolutions' operands rounded to half as the kernels' are
+@pytest.mark.parametrize("h,w", [(45, 46), (34, 57)])
+def test_vae_decode_of_a_width_no_tile_divides(gpu, h, w):
+    base = 96
     ref = R.Vae(base, seed=5, mean=MEAN, std=STD)
     vae = M.Vae(base, mean=MEAN, std=STD)
     vae.init_random(5)
