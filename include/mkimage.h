@@ -146,6 +146,10 @@ mk_status mk_gemm_grouped(const mk_gemm_args* a, uint32_t count, void* stream);
  * so they may run concurrently. No counterpart in the reference. */
 #define MK_GEMM_WAIT_LIMIT (1u << 26)
 mk_status mk_gemm_set_wait_limit(uint32_t polls);
+/* The plan of a launch on a device of cus compute units, without running it (host only; a test hook): out[0] x out[1] rows
+ * x channels a tile, out[2] workgroups a tile's k steps are split over (1: whole tiles). No counterpart in the
+ * reference. */
+mk_status mk_gemm_plan(const mk_gemm_args* a, uint32_t count, uint32_t cus, uint32_t* out);
 
 /* 3x3 convolution, stride 1, zero padding 1 (the VAE decoder's conv, src/image/engine.cpp:732-746, 907-947), as one
  * GEMM over the padded pixel grid (implicit im2col on MFMA) in IEEE half operands with fp32 sums, as the reference

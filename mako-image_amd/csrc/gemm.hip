@@ -2049,11 +2049,11 @@ template <int EK> void launch_reduce(const GemmG& G, const float* ws, uint32_t s
     gemm_reduce_kernel<EK><<<cdiv(items, 256), 256, 0, s>>>(G, ws, splits, slab, items);
 }
 
-// A split launch of `plan.splits` k ranges a 128 x 128 tile; `done` is left false when the stream is being captured or
-// no slab buffer can be had (a captured launch must not own memory another launch may use): the caller then launches
-// whole tiles.
-mk_status launch_split(GemmP* p, uint32_t count, const GemmPlan& plan, int ek, bool f8, bool f16, uint32_t cus,
-                       hipStream_t s, bool& done)
+// A split launch of `plan.splits` k ranges a 128 x 128 tile, at most one workgroup a CU and slabs that fit a buffer
+// (gemm_plan); `done` is left false when the stream is being captured or no slab buffer can be had (a captured launch
+// must not own memory another launch may use): the caller then launches whole tiles.
+mk_status launch_split(GemmP* p, uint32_t count, const GemmPlan& plan, int ek, bool f8, bool f16, hipStream_t s,
+                       bool& done)
 {
     done = false;
     if (capturing(s))
@@ -2073,8 +2073,6 @@ mk_status launch_split(GemmP* p, uint32_t count, const GemmPlan& plan, int ek, b
     }
     const uint32_t N = p[0].N, splits = uint32_t(plan.splits);
     const uint64_t slab = uint64_t(rows) * N;
-    if (slab * splits * 4 > kSplitBytes)
-        return MK_OK;
     std::lock_guard<std::mutex> lock(g_sk_mutex);
     SplitWork* W = split_acquire(g_split[dev], s);
     if (!W)
@@ -2094,17 +2092,12 @@ mk_status launch_split(GemmP* p, uint32_t count, const GemmPlan& plan, int ek, b
     }
     P.tiles0 = count > 1 ? p[0].tiles_m * p[0].tiles_n * p[0].batch : tiles;
     const uint32_t wgs = tiles * splits;
-    constexpr int H = EK_STORE | EK_F16;
     if (f8)
         gemm_split_kernel<128, 128, true, EK_STORE, 4><<<wgs, 256, 0, s>>>(P, splits, tiles, slab);
-    else if (f16 && wgs <= cus)
-        gemm_split_kernel<128, 128, false, H | EK_DEEP, 4><<<wgs, 256, 0, s>>>(P, splits, tiles, slab);
     else if (f16)
-        gemm_split_kernel<128, 128, false, H, 4><<<wgs, 256, 0, s>>>(P, splits, tiles, slab);
-    else if (wgs <= cus)
-        gemm_split_kernel<128, 128, false, EK_STORE | EK_DEEP, 4><<<wgs, 256, 0, s>>>(P, splits, tiles, slab);
+        gemm_split_kernel<128, 128, false, EK_STORE | EK_F16 | EK_DEEP, 4><<<wgs, 256, 0, s>>>(P, splits, tiles, slab);
     else
-        gemm_split_kernel<128, 128, false, EK_STORE, 4><<<wgs, 256, 0, s>>>(P, splits, tiles, slab);
+        gemm_split_kernel<128, 128, false, EK_STORE | EK_DEEP, 4><<<wgs, 256, 0, s>>>(P, splits, tiles, slab);
     MK_HIP(hipGetLastError());
     if (ek == EK_STORE)
         launch_reduce<EK_STORE>(G, ws, splits, slab, rows, s);
@@ -2516,7 +2509,9 @@ GemmPlan gemm_plan(const mk_gemm_args* a, uint32_t n, uint32_t cus, bool conv, b
     uint64_t rows = 0;
     for (uint32_t i = 0; i < n; ++i)
         rows += uint64_t(a[i].M) * a[i].batch;
-    if (!conv && N % 128 == 0 && rows < 1024) {
+    const bool f16_act = a[0].w_dtype == MK_F16 &&
+                         gemm_detail::epi_kind(a[0].epilogue) == gemm_detail::EK_ACT; // (the dispatch refuses these)
+    if (!conv && !f16_act && N % 128 == 0 && rows < 1024) {
         const uint64_t cap = cus / std::max<uint64_t>(1, tiles_of(128, 128));
         const double slab = double(rows) * N * 4, whole = (f8 ? 0.6 : 0.42) * double(kt);
         double least = whole;
@@ -2586,9 +2581,9 @@ extern "C" mk_status mk_gemm_grouped(const mk_gemm_args* a, uint32_t count, void
     if (n == 1 && p[0].N == 64 && ek == EK_STORE && !f8 && !p[0].wscale &&
         uint64_t(cdiv(p[0].M, 32)) * p[0].batch <= rounds64 * uint64_t(cus > 0 ? cus : 1))
         return launch_n64(p[0], a[0].w_dtype == MK_F16, s);
-    if (plan.splits > 1 && !(ek == EK_ACT && a[0].w_dtype == MK_F16)) {
+    if (plan.splits > 1) {
         bool done = false;
-        MK_TRY(launch_split(p, n, plan, ek, f8, a[0].w_dtype == MK_F16, uint32_t(cus > 0 ? cus : 1), s, done));
+        MK_TRY(launch_split(p, n, plan, ek, f8, a[0].w_dtype == MK_F16, s, done));
         if (done)
             return MK_OK;
     }
@@ -2690,6 +2685,23 @@ extern "C" mk_status mk_gemm_grouped(const mk_gemm_args* a, uint32_t count, void
 }
 
 extern "C" mk_status mk_gemm(const mk_gemm_args* a, void* stream) { return mk_gemm_grouped(a, 1, stream); }
+
+extern "C" mk_status mk_gemm_plan(const mk_gemm_args* a, uint32_t count, uint32_t cus, uint32_t* out)
+{
+    if (!a || !out || !count || count > 2 || !cus)
+        return fail(MK_ERR_ARG, "gemm_plan: null argument, no compute units or not 1 or 2 problems");
+    for (uint32_t i = 0; i < count; ++i) {
+        GemmP p;
+        MK_TRY(prepare(&a[i], p));
+        if (!a[i].M || !a[i].batch)
+            return fail(MK_ERR_ARG, "gemm_plan: empty problem");
+    }
+    const GemmPlan plan = gemm_plan(a, count, cus);
+    out[0] = uint32_t(plan.bm);
+    out[1] = uint32_t(plan.bn);
+    out[2] = uint32_t(plan.splits > 1 ? plan.splits : 1);
+    return MK_OK;
+}
 
 extern "C" mk_status mk_gemm_set_wait_limit(uint32_t polls)
 {

@@ -89,6 +89,7 @@ _SIGS = {
     "mk_gemm": (_i, [C.POINTER(GemmArgs), _vp]),
     "mk_gemm_grouped": (_i, [_vp, _u32, _vp]),
     "mk_gemm_set_wait_limit": (_i, [_u32]),
+    "mk_gemm_plan": (_i, [_vp, _u32, _u32, C.POINTER(_u32)]),
     "mk_gemv": (_i, [_vp, _u32, _u32, _vp, _vp, _u32, _vp, _i, _vp]),
     "mk_ln_modulate": (_i, [_vp, _u32, _u32, _vp, _vp, _i64, _u32, _u32, _f, _vp, _vp]),
     "mk_gate_add": (_i, [_vp, _vp, _u32, _u32, _u32, _vp, _i64, _u32, _u32, _i, _vp]),

@@ -128,3 +128,31 @@ def test_vae_up_plan():
     # rounds are the device's: twice the image on twice the units, half of it on half
     assert plan(608, 208, 384, 512) == plan(304, 208, 384, 256) == plan(152, 208, 384, 128) == 1
     assert mkimage.lib().mk_vae_up_plan(304, 208, 100, 256, ctypes.byref(ctypes.c_uint32())) == 1
+
+
+def _plan(rows, n, k, epi=0, w_dtype=mkimage.BF16, cus=256):
+    g = mkimage.GemmArgs()
+    g.a = g.w = g.c = g.gate = g.wscale = 4096  # (not read)
+    g.M, g.N, g.K, g.lda, g.ldc, g.batch = rows, n, k, k, n, 1
+    g.w_dtype, g.c_dtype, g.epilogue = w_dtype, mkimage.F32, epi
+    out = (ctypes.c_uint32 * 3)()
+    mkimage.call("mk_gemm_plan", ctypes.byref(g), 1, cus, out)
+    return tuple(out)
+
+
+def test_gemm_plan_splits():
+    # below 1024 rows a tile's k steps are split while that is estimated faster, at most a workgroup a compute unit; never
+    # for an epilogue the weight type has not
+    assert _plan(77, 3072, 12288)[2] == 10 and _plan(320, 3072, 12288)[2] == 3
+    assert _plan(1023, 256, 12288)[2] > 1 and _plan(1024, 256, 12288)[2] == 1
+    assert _plan(1, 128, 832)[2] == 1 and _plan(1, 128, 896)[2] == 4  # 13 and 14 k steps
+    assert _plan(1, 128, 576, w_dtype=mkimage.FP8)[2] == 1 and _plan(1, 128, 640, w_dtype=mkimage.FP8)[2] == 4
+    assert _plan(512, 1280, 1280)[2] == 1
+    for rows, n, k in ((1, 128, 12288), (300, 640, 12288), (900, 1024, 12288), (1023, 1920, 8192)):
+        tiles = -(-rows // 128) * (n // 128)
+        for wdt in (mkimage.BF16, mkimage.FP8, mkimage.F16):
+            splits = _plan(rows, n, k, w_dtype=wdt)[2]
+            assert splits == 1 or (splits * tiles <= 256 and splits * rows * n * 4 <= 32 << 20)
+    for epi in (mkimage.EPI_GELU_TANH, mkimage.EPI_SILU):
+        assert _plan(77, 3072, 12288, epi)[2] > 1
+        assert _plan(77, 3072, 12288, epi, mkimage.F16)[2] == 1
