@@ -70,6 +70,15 @@ def gemm_args(A, W, *, bias=None, wscale=None, epi=M.EPI_STORE, c=None, c_dtype=
     return g
 
 
+def plan(Mr, N, K, epi, wdt):
+    """(rows, channels, workgroups over the k steps) of a launch's tiles on 256 compute units."""
+    g = gemm_args(M.Dev(16), M.Dev(16), M_=(Mr, N, K), lda=K, ldc=N, epi=epi, w_dtype=wdt)
+    g.c = g.gate = g.wscale = g.a  # (not read)
+    out = (C.c_uint32 * 3)()
+    M.call("mk_gemm_plan", C.byref(g), 1, 256, out)
+    return tuple(out)
+
+
 def gemm_grouped(*args):
     arr = (M.GemmArgs * len(args))(*args)
     M.call("mk_gemm_grouped", C.cast(arr, C.c_void_p), len(args), None)
@@ -286,14 +295,17 @@ def test_gemm_heads_epilogue(gpu, rng, mode, row0, q_row0, k_scale, odt):
 
 
 # Few rows and long K: the k steps split over workgroups, the slabs added and put through the epilogue by a second
-# kernel. One row, rows that end inside a tile, the most rows that split, uneven k ranges (K of 9 to 192 k steps), every
-# epilogue, weight type and output type, against the oracle's product; a second launch repeats the bits.
-@pytest.mark.parametrize("Mr,N,K", [(1, 128, 2048), (77, 384, 6144), (512, 256, 1600), (130, 128, 12288)])
+# kernel. One row, rows that end inside a tile, the most rows that split, uneven k ranges (K of 14 to 192 k steps, 14 the
+# fewest that split), every epilogue, weight type and output type, against the oracle's product; a second launch
+# repeats the bits.
+@pytest.mark.parametrize("Mr,N,K", [(1, 128, 2048), (77, 384, 6144), (512, 256, 1600), (130, 128, 12288),
+                                    (1, 128, 896), (1023, 128, 1600)])
 @pytest.mark.parametrize("epi,wdt", [(M.EPI_STORE, M.BF16), (M.EPI_STORE, M.FP8), (M.EPI_STORE, M.F16),
                                      (M.EPI_GATE_TANH, M.BF16), (M.EPI_GATE_ADD, M.FP8), (M.EPI_ADD, M.F16),
                                      (M.EPI_GELU_TANH, M.BF16), (M.EPI_SILU, M.FP8), (M.EPI_SWIGLU, M.BF16),
                                      (M.EPI_GEGLU, M.F16), (M.EPI_PAIR_SUM, M.F16)])
 def test_gemm_split_k(gpu, rng, Mr, N, K, epi, wdt):
+    assert plan(Mr, N, K, epi, wdt)[2] > 1
     rnd, bits = (R.f16_round, M.f16_bits) if wdt == M.F16 else (R.bf16_round, M.bf16_bits)
     A = rnd(rng.standard_normal((Mr, K)).astype(np.float32))
     Wf = rng.standard_normal((N, K)).astype(np.float32) * 0.03
@@ -402,8 +414,9 @@ def test_gemm_split_k_grouped_on_many_streams(gpu, rng):
 
 
 # 64 output channels take a kernel of their own: row counts that end inside its 32-token tiles, K of fewer k steps than
-# its 4 waves, of whole and of cut rounds of its 3 stages, strides, batch items and each output type
-@pytest.mark.parametrize("Mr,K", [(1, 64), (31, 192), (33, 832), (64, 768), (300, 3072), (8200, 1536)])
+# its 4 waves, of whole and of cut rounds of its 3 stages, strides, batch items and each output type; 258 workgroups, one
+# more than the units hold, and 514, two rounds and more, which take 256 x 64 tiles again
+@pytest.mark.parametrize("Mr,K", [(1, 64), (31, 192), (33, 832), (64, 768), (300, 3072), (4100, 1536), (8200, 1536)])
 @pytest.mark.parametrize("wdt,cdt", [(M.BF16, M.F32), (M.BF16, M.BF16), (M.F16, M.F16)])
 def test_gemm_64_channels(gpu, rng, Mr, K, wdt, cdt):
     B, N, lda, ldc = 2, 64, K + 64, 72
@@ -1404,10 +1417,12 @@ def test_attention_general_scale_range(gpu, rng, dtype, d, scale, mag, block):
 
 
 # Launches of at most one tile a CU on 128-channel tiles run deep-staged (4 LDS stages for 128 x 128 tiles, 3 for
-# 256 x 128): K of 1 to 20 k steps covers the prologue, whole unrolled rounds and every remainder length.
+# 256 x 128): K of 1 to 20 k steps covers the prologue, whole unrolled rounds and every remainder length (256 rows of 20 k
+# steps split them; 1024 rows do not).
 @pytest.mark.parametrize("K", [64, 128, 192, 256, 320, 448, 1280])
-@pytest.mark.parametrize("Mr,N", [(256, 256), (8192, 640)])  # 4 tiles of 128 x 128; 160 of 256 x 128
+@pytest.mark.parametrize("Mr,N", [(256, 256), (1024, 256), (8192, 640)])  # 4 and 16 tiles of 128 x 128; 160 of 256 x 128
 def test_gemm_deep_staged_lone_tiles(gpu, rng, Mr, N, K):
+    assert plan(Mr, N, K, M.EPI_STORE, M.BF16) == (256 if Mr == 8192 else 128, 128, 4 if (Mr, K) == (256, 1280) else 1)
     A = rng.standard_normal((Mr, K)).astype(np.float32)
     W = R.bf16_round(rng.standard_normal((N, K)).astype(np.float32) * 0.05)
     b = rng.standard_normal(N).astype(np.float32) * 0.3
