@@ -232,7 +232,7 @@ mk_status mk_rms_norm(const float* x, uint32_t rows, uint32_t n, const float* w,
 /* layer_norm with gamma, beta (sdxl.cpp:425-437): x fp32, y bf16 */
 mk_status mk_layer_norm(const float* x, uint32_t rows, uint32_t n, const float* g, const float* b, float eps, void* y,
                         void* stream);
-/* group_norm over channels-last [batch][rows][c], `groups` groups, affine; y bf16 */
+/* group_norm over channels-last [batch][rows][c], `groups` groups, affine; y bf16 (refused on a stream under capture) */
 mk_status mk_group_norm(const float* x, uint32_t batch, uint32_t rows, uint32_t c, uint32_t groups, const float* g,
                         const float* b, float eps, void* y, void* stream);
 /* mk_group_norm without allocating: no counterpart in the reference; for callers that cannot allocate device memory

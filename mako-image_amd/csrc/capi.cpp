@@ -34,6 +34,16 @@ void forget_stream(const void* stream)
     g_streams.erase(std::remove(g_streams.begin(), g_streams.end(), stream), g_streams.end());
 }
 
+bool capturing(const void* stream)
+{
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(static_cast<hipStream_t>(const_cast<void*>(stream)), &cap) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return cap != hipStreamCaptureStatusNone;
+}
+
 void set_error(const std::string& msg) { g_error = msg; }
 
 mk_status fail(mk_status s, const std::string& msg)

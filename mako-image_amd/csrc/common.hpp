@@ -73,6 +73,8 @@ mk_status gemm_take_error(const void* stream, bool all = false);
 void adopt_stream(const void* stream);
 bool known_stream(const void* stream);
 void forget_stream(const void* stream);
+// Whether a stream is being captured into a graph (or cannot be asked because another one is).
+bool capturing(const void* stream);
 // To be called before a stream is destroyed: waits for its last stream-K, split-K and group norm launches and frees their
 // workspaces for other streams (an event must not be asked after the stream it was recorded on is gone).
 void release_stream(const void* stream);

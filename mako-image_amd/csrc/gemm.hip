@@ -1864,16 +1864,6 @@ bool event_done(hipEvent_t done)
     return e == hipSuccess;
 }
 
-bool capturing(hipStream_t s)
-{
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
-        (void)hipGetLastError();
-        return true;
-    }
-    return cap != hipStreamCaptureStatusNone;
-}
-
 // Lets this thread allocate and ask events while another stream is being captured (in the default mode such a call ends
 // that stream's capture; none of them concerns it).
 struct RelaxedCapture {

@@ -987,7 +987,8 @@ static mk_status group_norm_run(const float* x, uint32_t batch, uint32_t rows, u
 // steady-state call allocates nothing. A call's stream first waits for the event of the buffer's previous user unless
 // that was the same stream (the same handle, of a known_stream), and records it after its own kernels: calls on
 // different streams take turns on the buffer. A stream that is about to be destroyed gives the buffer back
-// (group_norm_release_stream): the event of a destroyed stream must not be waited for.
+// (group_norm_release_stream): the event of a destroyed stream must not be waited for. A capture is refused: a graph's
+// replays would take no turns and keep a buffer that a later call may free.
 struct GnScratch {
     int dev = -1;
     char* p = nullptr;
@@ -1019,6 +1020,8 @@ mk_status group_norm_to(const float* x, uint32_t batch, uint32_t rows, uint32_t 
     int dev = 0;
     MK_HIP(hipGetDevice(&dev));
     const hipStream_t s = S(stream);
+    if (capturing(s))
+        return fail(MK_ERR_DEVICE, "group_norm: its scratch cannot go into a graph (mk_group_norm_noalloc has none)");
     std::lock_guard<std::mutex> lock(g_gn_mutex);
     GnScratch* w = nullptr;
     for (GnScratch& e : g_gn)

@@ -245,3 +245,26 @@ def test_small_gemms_during_another_streams_capture(gpu):
     assert hip.hipGraphExecDestroy(run) == 0 and hip.hipGraphDestroy(graph) == 0
     for s in (cap, *others):
         M.call("mk_stream_destroy", s)
+
+
+def test_group_norm_is_refused_under_capture(gpu):
+    # its scratch is shared with later calls, which may free it: a graph must not keep it, also where the capturing
+    # stream was the scratch's last user
+    hip = C.CDLL("libamdhip64.so.7")
+    work = Small(0)
+    h, graph = C.c_void_p(), C.c_void_p()
+    M.call("mk_stream_create", C.byref(h))
+    work.launch(h.value, work.out())
+    M.sync()
+    want = work.read()[0][-1]
+    y = M.Dev(want.nbytes)
+    args = (work.x.p, *GN, work.g.p, work.gb.p, 1e-6, y.p, h.value)
+    assert hip.hipStreamBeginCapture(h, 0) == 0
+    status = M.lib().mk_group_norm(*args)
+    assert hip.hipStreamEndCapture(h, C.byref(graph)) == 0
+    assert hip.hipGraphDestroy(graph) == 0
+    assert status != 0 and b"graph" in M.lib().mk_last_error()
+    M.call("mk_group_norm", *args)
+    M.sync()
+    assert np.array_equal(y.to_array(np.uint16, want.shape), want)
+    M.call("mk_stream_destroy", h.value)
