@@ -1889,7 +1889,7 @@ mk_status sk_acquire(SkDevice& D, hipStream_t s, size_t need, uint32_t nflags, S
     for (auto& w : D.pool)
         if (w->last == s && w->ws_bytes >= need && w->nflags >= nflags)
             pick = w.get();
-    if (pick && !pick->known && !capturing(s)) // (a capture cannot wait for an event of before it)
+    if (pick && !pick->known)
         MK_TRY(wait_done(s, pick->done));
     if (!pick)
         for (auto& w : D.pool)
@@ -2132,7 +2132,9 @@ mk_status launch(GemmP* p, uint32_t count, const GemmPlan& plan, hipStream_t s)
             D.cus = n > 0 ? uint32_t(n) : 1;
         }
         const uint32_t grid = D.cus;
-        if (plan.sk && plan.dp % grid == 0 && plan.dp < tiles) {
+        // under capture whole tiles: a graph's replays would repeat one epoch, whose flags the replay before has set, and
+        // keep a workspace that other launches use
+        if (plan.sk && plan.dp % grid == 0 && plan.dp < tiles && !capturing(s)) {
             MK_TRY(sk_check(D, s, false));
             SkP sk{};
             sk.total = tiles;

@@ -700,8 +700,8 @@ def _sk_problem(rng, K=6144):
                 gd=dev(gt))
 
 
-def _sk_launch(P, stream=None):
-    cs = [dev(x) for x in P["X"]]
+def _sk_launch(P, stream=None, cs=None):
+    cs = cs or [dev(x) for x in P["X"]]
     args = [gemm_args(a, P["Wd"], bias=P["bd"], c=c, epi=M.EPI_GATE_ADD, M_=(Mr, P["N"], P["K"]), lda=P["K"],
                       ldc=P["N"], gate=P["gd"]) for a, c, Mr in zip(P["Ad"], cs, P["shapes"])]
     arr = (M.GemmArgs * 2)(*args)
@@ -769,6 +769,39 @@ def test_gemm_stream_k_after_its_stream_is_destroyed(gpu, rng):
             got = [fetch(c, (Mr, P["N"])) for c, Mr in zip(got, P["shapes"])]
             want = want or got
             assert all(np.array_equal(a, b) for a, b in zip(got, want))
+
+
+def test_gemm_stream_k_shape_in_a_graph(gpu, rng):
+    # a captured launch of a stream-K shape runs whole tiles (a replay cannot tell its partials from the last replay's):
+    # every replay's result on new inputs, with eager stream-K launches between, against the oracle
+    hip = C.CDLL("libamdhip64.so.7")
+    P = [_sk_problem(np.random.default_rng(s)) for s in (31, 32)]
+    h, graph, run = C.c_void_p(), C.c_void_p(), C.c_void_p()
+    M.call("mk_stream_create", C.byref(h))
+    _sk_launch(P[0], h.value)
+    M.sync()
+    cs = [dev(x) for x in P[0]["X"]]
+    assert hip.hipStreamBeginCapture(h, 0) == 0
+    _sk_launch(P[0], h.value, cs)
+    assert hip.hipStreamEndCapture(h, C.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(C.byref(run), graph, None, None, 0) == 0
+    for rep in range(3):
+        p = P[rep % 2]
+        for i, c in enumerate(cs):
+            M.call("mk_memcpy_h2d", c.p, p["X"][i].ctypes.data, p["X"][i].nbytes)
+            a = M.bf16_bits(p["A"][i])
+            M.call("mk_memcpy_h2d", P[0]["Ad"][i].p, a.ctypes.data, a.nbytes)
+        assert hip.hipGraphLaunch(run, h) == 0
+        M.call("mk_stream_synchronize", h.value)
+        for i, (c, Mr) in enumerate(zip(cs, p["shapes"])):
+            got = fetch(c, (Mr, p["N"]))
+            rows = np.sort(rng.choice(Mr, 24, replace=False))
+            want = p["X"][i][rows].astype(np.float64) + P[0]["gt"] * R.gemm(p["A"][i][rows], P[0]["W"], P[0]["b"])
+            assert maxrel(got[rows], want) < 1e-5
+        _sk_launch(P[1], h.value)
+        M.sync()
+    assert hip.hipGraphExecDestroy(run) == 0 and hip.hipGraphDestroy(graph) == 0
+    M.call("mk_stream_destroy", h.value)
 
 
 def test_gemm_stream_k_gave_up_wait_is_reported(gpu, rng):
