@@ -130,8 +130,11 @@ typedef struct mk_gemm_args {
 
 /* proj (the reference's GEMM, engine.cpp:768 / qwen_image.cpp:196-288): C = A W^T with the fused epilogue.
  * K % 64 == 0, N % 64 == 0. Launches of fewer than 1024 rows may split their k steps over workgroups into fp32 slabs of the
- * library's (at most 8 x 32 MB a device, one a stream; whole tiles when the stream is being captured): the sums then run
- * in another, fixed order than a larger launch's. */
+ * library's (at most 8 x 32 MB a device, one a stream), and long launches their last wave's (stream-K, below). The sums
+ * then run in another order, fixed for the launch's shape: a row's last bits can depend on how many rows share the
+ * launch. On a stream under capture, and while no slabs can be had, a launch runs whole tiles: a graph's replays agree with
+ * each other, and with the eager launch to fp32 rounding. A stream that is not the null stream, an engine's, a VAE's or
+ * mk_stream_create's (hipStreamPerThread among them) pays an event a split launch. */
 mk_status mk_gemm(const mk_gemm_args* a, void* stream);
 /* count (1 or 2) GEMMs of equal N, K, weight dtype and epilogue kind in one launch: the dual-stream blocks' image and
  * text projections, whose separate launches would leave most of the chip idle on the text's few tiles. Each problem

@@ -198,8 +198,9 @@ __device__ inline void epi_slice(const GemmP& p, const float* st, int ld, int to
     }
     if constexpr (EK == EK_RMWUP) {
         // x + v (the convolution's ADD) goes to the four pixels (2 y + dy, 2 x + dx) of the nearest 2x grid, 16-bit;
-        // the residual itself is not stored (its next reader is the upsampling). Tiles over the pixels only: every
-        // row of the slice is a pixel of image row y; else the row's pixel by an integer division, ring rows left out.
+        // the residual itself is not stored (its next reader is the upsampling). Where the tiles cover the pixels only
+        // (conv_w) every row of the slice is a pixel of one image row; over the padded rows a row's pixel comes from an
+        // integer division, and ring rows are left out.
         const float* c = static_cast<const float*>(p.c) + ch;
         const uint32_t pw = p.conv_pw, gh = p.M / pw, gy0 = uint32_t(tok0) / pw, ld2 = p.norm_ld;
         uint16_t* up = p.norm_out + ch;
@@ -2416,7 +2417,7 @@ mk_status gemm_take_error(const void* stream, bool all)
 // 0.66, 256 x 64 0.62, 128 x 128 0.67 for a pair of tiles (two workgroups share a CU: 64 KB of LDS each), so a wave of
 // 128 x 128 tiles is 2 per CU and an odd last tile costs half a pair; ties keep the larger tile. Convolutions also
 // have 256 x 192 tiles (8 waves, 0.78), for their 192- and 384-channel layers, and 128 x 96 tiles (4 waves on
-// 16 x 16 x 32, two workgroups a CU) for output channels that are an odd multiple of 96. The heads epilogue
+// 16 x 16 x 32, two workgroups a CU) for output channels that are a multiple of 96. The heads epilogue
 // takes 256 x 256 or 128 x 128 tiles for 128-dim heads and 128-channel tiles for 64-dim heads; half-weight convolutions
 // 256-token tiles.
 // 256 x 256 tiles use stream-K when whole waves leave at least 5% of the last wave's workgroups idle and
@@ -2480,7 +2481,9 @@ GemmPlan gemm_plan(const mk_gemm_args* a, uint32_t n, uint32_t cus, bool conv, b
     consider(256, 128, 0.66);
     if (conv)
         consider(256, 192, 0.78);
-    if (conv && (N % 64 || by_row)) // 96 output channels (and odd multiples of 96) take 128 x 96 tiles, nothing else
+    // 128 x 96 tiles: all there is for output channels that are odd multiples of 96, and where conv_kernel takes them for
+    // other multiples too
+    if (conv && (N % 64 || by_row))
         consider(128, 96, 0.5);
     if (narrow_ok)
         consider(256, 64, 0.62);
@@ -2497,7 +2500,8 @@ GemmPlan gemm_plan(const mk_gemm_args* a, uint32_t n, uint32_t cus, bool conv, b
     // 3072 x 12288 120 -> 24 (10), 64 x 3072 x 3584 19.7 -> 12.7 (6), 77 x 12288 x 3072 33 -> 27 (2), f16 512 x 1280 x
     // 5120 34 -> 19 (4), 600 x 3072 x 12288 110 -> 72 (2), 960 x 1280 x 5120 35 -> 23 (3); 512 x 1280 x 1280 stays whole
     // (13.6 against 14.0 in two), so does 640 x 3072 x 3584 (23.6 against 27.0). 1024 rows and more stay whole, so that
-    // the parts of an image's rows launched apart get the bits of one launch.
+    // the parts of an image's rows launched apart get the bits of one launch: 1024 x 1280 x 5120 gives up 36 -> 26 us for
+    // that, 1100 x 3072 x 12288, 2048 x 1280 x 5120 and 3952 x 640 x 2560 nothing (too many tiles to split).
     uint64_t rows = 0;
     for (uint32_t i = 0; i < n; ++i)
         rows += uint64_t(a[i].M) * a[i].batch;

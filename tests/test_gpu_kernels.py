@@ -2,6 +2,7 @@
 ABI on seeded inputs, against the oracle (oracle/mkref.cpp). Index / byte work (patchify, the RNG fill, fp8 codes,
 layouts) is bit-exact; floating point is within the stated tolerance."""
 import ctypes as C
+import threading
 
 import numpy as np
 import pytest
@@ -752,6 +753,37 @@ def test_gemm_stream_k_on_two_streams_at_once(gpu, rng):
         M.sync()
         for st in streams:
             M.call("mk_stream_destroy", st)
+
+
+def test_gemm_stream_k_on_per_thread_streams(gpu, rng):
+    # hipStreamPerThread is one handle, a stream of its own in each thread: one thread's partials are not another's
+    P = [_sk_problem(np.random.default_rng(s)) for s in (41, 42)]
+    want, outs, errors = [], [], []
+    for p in P:
+        cs = _sk_launch(p)
+        M.sync()
+        want.append([fetch(c, (Mr, p["N"])) for c, Mr in zip(cs, p["shapes"])])
+        outs.append([[dev(x) for x in p["X"]] for _ in range(4)])
+    start = threading.Barrier(2)
+
+    def run(p, sets):
+        try:
+            start.wait()
+            for cs in sets:
+                _sk_launch(p, 2, cs)
+            M.call("mk_stream_synchronize", 2)
+        except Exception as e:  # noqa: BLE001
+            errors.append(e)
+
+    threads = [threading.Thread(target=run, args=a) for a in zip(P, outs)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors
+    for p, w, sets in zip(P, want, outs):
+        for cs in sets:
+            assert all(np.array_equal(fetch(c, (Mr, p["N"])), a) for c, Mr, a in zip(cs, p["shapes"], w))
 
 
 def test_gemm_stream_k_after_its_stream_is_destroyed(gpu, rng):
