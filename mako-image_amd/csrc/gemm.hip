@@ -1953,8 +1953,9 @@ mk_status sk_check(SkDevice& D, hipStream_t s, bool all)
 // follow each other on its own buffer and streams never share one. Where the handle alone does not say that it is the
 // same stream (known_stream), a launch records an event and the next one on that handle waits for it (2.8 us a launch;
 // the FFN over 77 rows, two of them, 52.5 -> 58.1 us). A stream without a buffer takes a free one, one whose event is
-// reached, a new one, or the least recently used one behind its event: the stream waits for that, not the host. Once
-// more streams than buffers have come by, every launch records its event. A destroyed stream's buffer is given back by
+// reached or whose stream is idle (an allocation takes 30 to 400 us, which the first step of every new engine paid), a
+// new one, or the least recently used one behind its event: the stream waits for that, not the host. Once more streams
+// than buffers have come by, every launch records its event. A destroyed stream's buffer is given back by
 // release_stream. (32 MB of slabs stay in the memory-side cache between the two kernels.) Locked with g_sk_mutex over
 // both launches.
 constexpr size_t kSplitBytes = size_t(32) << 20, kSplitPool = 8;
@@ -1972,6 +1973,20 @@ struct SplitDevice {
     std::vector<SplitWork> pool;
 };
 SplitDevice g_split[kMaxDevices];
+
+// Whether the last launch on buffer w is complete: its event is reached or, where it left none, its stream (a
+// known_stream, so alive) has nothing left to do.
+bool split_idle(const SplitWork& w)
+{
+    if (w.marked)
+        return event_done(w.done);
+    if (capturing(w.owner))
+        return false;
+    const hipError_t e = hipStreamQuery(w.owner);
+    if (e != hipSuccess && e != hipErrorNotReady)
+        (void)hipGetLastError();
+    return e == hipSuccess;
+}
 
 // Stream s after the last launch on buffer w: false where that cannot be waited for now (it left no event, and its
 // stream is being captured).
@@ -2000,7 +2015,7 @@ SplitWork* split_acquire(SplitDevice& D, hipStream_t s)
         return nullptr;
     if (!pick)
         for (auto& w : D.pool)
-            if (!w.owned || (w.marked && event_done(w.done))) {
+            if (!w.owned || split_idle(w)) {
                 pick = &w;
                 break;
             }

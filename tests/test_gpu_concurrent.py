@@ -203,6 +203,34 @@ def test_split_launches_on_more_streams_than_slab_buffers_do_not_wait_for_the_de
         M.call("mk_stream_destroy", s)
 
 
+def test_streams_used_in_turn_share_a_slab_buffer(gpu):
+    # a new stream's first split launch takes an idle stream's buffer instead of allocating one
+    hip = C.CDLL("libamdhip64.so.7")
+
+    def free():
+        a, b = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(a), C.byref(b)) == 0
+        return a.value
+
+    work = Small(0)
+    handles = [C.c_void_p() for _ in range(5)]
+    for h in handles:
+        M.call("mk_stream_create", C.byref(h))
+    bufs = [work.out() for _ in handles]
+    work.launch(handles[0].value, bufs[0])
+    M.sync()
+    before = free()
+    for h, b in zip(handles[1:], bufs[1:]):
+        work.launch(h.value, b)
+        M.sync()
+    assert before - free() < 32 << 20
+    want, *rest = work.read()
+    for got in rest:
+        assert all(np.array_equal(a, b) for a, b in zip(got, want))
+    for h in handles:
+        M.call("mk_stream_destroy", h.value)
+
+
 def test_small_gemms_during_another_streams_capture(gpu):
     # one stream is being captured while others run split launches for the first time (they need slab buffers); the
     # captured launches, of sizes that split when they are not captured, run whole tiles, the same bits every replay
