@@ -96,7 +96,7 @@ template <> struct Elem<true> {
 // U: K carries the softmax scale in log2 units (scale 0 at the API), so the softmax needs no per-score multiply at all;
 // a general scale multiplies each S - m by c. (The general scale had a tile of its own, a max, a multiply-add and an
 // add a score between the MFMAs instead of in their shadow: 493 -> 463 us for 2 x 24 heads of 128 over 4352 rows; on
-// another box 427 us with its row sums by v_dot2 on the 16-bit probabilities, 420 with them in fp32, 1.11 PFLOP/s.)
+// another card 427 us with its row sums by v_dot2 on the 16-bit probabilities, 420 with them in fp32, 1.11 PFLOP/s.)
 // NW waves a workgroup (32 queries each): 4, or 2 for launches of few query blocks (64-dim heads), whose 64-query
 // workgroups then spread over every CU, four a CU.
 template <int D, bool U, bool F16, bool HOLE, int NW = 4>

@@ -1464,7 +1464,7 @@ __global__ __launch_bounds__(64 * NW, BM == 128 && !(EK & EK_DEEP) ? 2 : 1) __at
 // within each 64 bytes, so 16 rows at one chunk cover all banks. One barrier a step, between its second and third tap:
 // behind it the third tap's products read the next step's first fragments and refill this step's stage. The 96-channel
 // tiles take 256 pixels (64 a wave: 10 fragment reads for 24 products instead of 8 for 12, the LDS bound of 128 pixels)
-// with two stages where that leaves two rounds of them. Measured at 1024 x 1024, 96 channels, on one box: norm epilogue
+// with two stages where that leaves two rounds of them. Measured at 1024 x 1024, 96 channels, on one card: norm epilogue
 // 274 -> 226 us (280 on 128-pixel tiles), adding and norming the fp32 residual 334 -> 270 (HBM: 1.2 GB), from 192
 // channels 466 -> 430; at 512 x 512, 192 channels, adding and norming 292 -> 269, norm alone 189 -> 191. The fp32
 // residual and the 192-channel tiles' uncovered epilogue (one workgroup a CU) bound what is left.
